@@ -32,7 +32,7 @@
 extern "C" {
 #endif
 
-#define SLK_ABI_VERSION 16
+#define SLK_ABI_VERSION 17
 
 #if defined(__GNUC__)
 #define SLK_API __attribute__((visibility("default")))
@@ -211,6 +211,8 @@ SLK_API int slk_abi_version(void);
  *                         histograms and scatter) everywhere, 1 = the radix
  *                         sort by column wherever ncols <= 65535 (automatic:
  *                         there, for total_capacity >= 2^20)
+ *   SLK_TUNE_QUAD_RW      slk_spmm_quad: row quads per wave (3, 4, 6 or 8; with
+ *                         one half also 9 or 16)
  * Returns SLK_EINVAL for an unknown knob.                                   */
 enum slk_tune_knob {
     SLK_TUNE_SPMM_KERNEL = 0,
@@ -227,7 +229,8 @@ enum slk_tune_knob {
     SLK_TUNE_RIGL_TILE = 11,
     SLK_TUNE_DENSE_ROWS = 12,
     SLK_TUNE_TRANSPOSE_RADIX = 13,
-    SLK_TUNE_COUNT = 14
+    SLK_TUNE_QUAD_RW = 14,
+    SLK_TUNE_COUNT = 15
 };
 SLK_API int slk_set_tuning(int knob, int64_t value);
 
@@ -251,6 +254,54 @@ SLK_API int slk_spmm(const slk_csr* W, const float* X, int64_t K, int64_t N,
  * array of W->nrows floats.                                                 */
 SLK_API int slk_spmm_bias(const slk_csr* W, const float* X, int64_t K, int64_t N,
                   const float* bias, float* Y, void* stream);
+
+/* A matrix's row quads (slk_quad_build), the schedule of slk_spmm_quad: one
+ * per topology, valid while row_start, row_nnz and col_indices are unchanged
+ * (values may change). X's rows are cut into chunks of 252 (halves = 1) or 126
+ * (halves = 2). For quad q (rows 4q .. 4q + 3) and chunk c, count[c * nq + q]
+ * is the most live slots that one of the rows holds in the chunk (nq =
+ * ceil(nrows / 4)), and its max(1, ceil(count / 16)) windows lie at
+ * start[c * nq + q] on: window w is the 64 entries from 64 w on of
+ * offset (the slot's X row as a byte offset into the chunk's 256 x halves byte
+ * rows) and slot (its index into values; -1 = none), entry 16 r + i the i-th
+ * of row r. The windows of one quad follow each other chunk by chunk. used[nq]
+ * is the number of windows; used[q] quad q's first. */
+typedef struct slk_quads {
+    const int32_t* start;
+    const uint8_t* count;
+    const uint32_t* offset;
+    const int32_t* slot;
+    const int32_t* used;
+    int64_t n_windows; /* allocated; a call's value buffer holds 64 per window */
+    int64_t halves;
+} slk_quads;
+
+/* Windows to allocate for W's quads, and X chunks of a matrix of ncols
+ * columns; 0 for an empty matrix or halves other than 1 and 2.              */
+SLK_API int64_t slk_quad_windows(const slk_csr* W, int64_t halves);
+SLK_API int64_t slk_quad_chunks(int64_t ncols, int64_t halves);
+
+/* Halves (1 or 2) of the quads that slk_spmm_quad would run W with on N columns,
+ * 0 where slk_spmm (estimated from W's capacity, shape and N) is about as fast
+ * or faster, W has heavy or dense rows, or a slk_spmm knob is set. Host only.  */
+SLK_API int64_t slk_quad_halves(const slk_csr* W, int64_t N);
+
+/* Builds W's quads on the device: three launches, no host read. With
+ * nq = ceil(nrows / 4) and nc = slk_quad_chunks(ncols, halves) (at most 2048):
+ * ws holds nq * 4 * (nc + 1) words of scratch, start nc * nq, count nc * nq
+ * bytes, offset and slot 64 * n_windows, used nq + 1. perm (may be NULL): W is
+ * a transpose and perm its slot map (slk_transpose_fill); the slots stored are
+ * then perm[slot], indexes into the values of the matrix it was built from.  */
+SLK_API int slk_quad_build(const slk_csr* W, const int64_t* perm, int64_t halves, int32_t* ws,
+                   int64_t ws_words, int32_t* start, uint8_t* count, uint32_t* offset,
+                   int32_t* slot, int64_t n_windows, int32_t* used, void* stream);
+
+/* slk_spmm (slk_spmm_bias with a bias; NULL: none) through W's quads, the same
+ * bits, for N in [4, 2^22]. values is what the quads' slots index (W's own, or
+ * with perm those of the matrix that W is the transpose of; W->values is not
+ * read). val_ws is scratch of 64 * n_windows floats, 16-byte aligned.        */
+SLK_API int slk_spmm_quad(const slk_csr* W, const slk_quads* Q, const float* values, float* val_ws,
+                  const float* X, int64_t K, int64_t N, const float* bias, float* Y, void* stream);
 
 /* dW[s] = dot(dY[i,:], X[col[s],:]) for every live slot s of row i, and
  * dW[s] = 0 for every padding slot. Replaces `spmm_grad_w_simd` /

@@ -21,7 +21,7 @@ from pathlib import Path
 import torch
 
 LIB_PATH = Path(__file__).resolve().parent / "_lib" / "libsparsecore_amd.so"
-ABI_VERSION = 16
+ABI_VERSION = 17
 
 SLK_OK, SLK_EINVAL, SLK_EDEVICE = 0, 1, 2
 SLK_DW_SIMD, SLK_DW_SCALAR = 0, 1
@@ -69,6 +69,11 @@ EXPORTS = (
     "slk_rigl_mfma_probe",
     "slk_dense_rows_workspace_bytes",
     "slk_dense_mfma_probe",
+    "slk_quad_windows",
+    "slk_quad_chunks",
+    "slk_quad_halves",
+    "slk_quad_build",
+    "slk_spmm_quad",
 )
 
 RIGL_INFO_BYTES = 32  # per row, slk_rigl_count's info
@@ -78,7 +83,8 @@ DROP_GROW_NOALLOC_MAX_SLOTS = 1 << 21  # SLK_DROP_GROW_NOALLOC_MAX_SLOTS
 # Kernel-choice overrides (slk_set_tuning): knob numbers of enum slk_tune_knob.
 TUNE_KNOBS = {"spmm_kernel": 0, "spmm_h": 1, "spmm_rw": 2, "spmm_split": 3, "spmm_vec": 4,
               "sddmm_g": 5, "seg_lean": 6, "seg_group": 7, "transpose_tile": 8, "spmm_bin": 9,
-              "spmm_g": 10, "rigl_tile": 11, "dense_rows": 12, "transpose_radix": 13}
+              "spmm_g": 10, "rigl_tile": 11, "dense_rows": 12, "transpose_radix": 13,
+              "quad_rw": 14}
 
 BIN_MAX_CHUNKS = 960  # SLK_BIN_MAX_CHUNKS
 
@@ -122,6 +128,20 @@ class CsrView(ctypes.Structure):
         ("n_dense_rows", ctypes.c_int64),
         ("dense_ws", ctypes.c_void_p),
         ("seg_dense_rows", ctypes.c_int64),
+    ]
+
+
+class QuadView(ctypes.Structure):
+    """Mirror of ``slk_quads`` (include/sparsecore_amd.h)."""
+
+    _fields_ = [
+        ("start", ctypes.c_void_p),
+        ("count", ctypes.c_void_p),
+        ("offset", ctypes.c_void_p),
+        ("slot", ctypes.c_void_p),
+        ("used", ctypes.c_void_p),
+        ("n_windows", ctypes.c_int64),
+        ("halves", ctypes.c_int64),
     ]
 
 
@@ -169,6 +189,14 @@ def _declare(lib) -> None:
     lib.slk_seg_list_workspace_bytes.argtypes = [_csrp, _i64]
     lib.slk_seg_list_build.argtypes = [_csrp, _i64, _i64, _vp, _i64, _vp, _vp, _vp, _i64, _vp,
                                        _vp]
+    for fn in (lib.slk_quad_windows, lib.slk_quad_chunks, lib.slk_quad_halves):
+        fn.restype = _i64
+    lib.slk_quad_windows.argtypes = [_csrp, _i64]
+    lib.slk_quad_chunks.argtypes = [_i64, _i64]
+    lib.slk_quad_halves.argtypes = [_csrp, _i64]
+    lib.slk_quad_build.argtypes = [_csrp, _vp, _i64, _vp, _i64, _vp, _vp, _vp, _vp, _i64, _vp, _vp]
+    lib.slk_spmm_quad.argtypes = [_csrp, ctypes.POINTER(QuadView), _vp, _vp, _vp, _i64, _i64, _vp,
+                                  _vp, _vp]
     lib.slk_phase_bounds_build.argtypes = [_csrp, _i64, _vp, _vp]
     lib.slk_set_tuning.argtypes = [ctypes.c_int, _i64]
     lib.slk_rigl_norms.argtypes = [_vp, _i64, _vp, _i64, _i64, _vp, _vp, _vp]
@@ -192,7 +220,8 @@ def _declare(lib) -> None:
     sized = ("slk_last_error", "slk_abi_version", "slk_transpose_workspace_bytes",
              "slk_drop_grow_workspace_bytes", "slk_rigl_bound_factor", "slk_rigl_partial_factor",
              "slk_dense_grad_approx_workspace_bytes",
-             "slk_seg_list_capacity", "slk_seg_list_workspace_bytes")
+             "slk_seg_list_capacity", "slk_seg_list_workspace_bytes", "slk_quad_windows",
+             "slk_quad_chunks", "slk_quad_halves")
     for name in EXPORTS:
         if name not in sized:
             getattr(lib, name).restype = ctypes.c_int
@@ -391,6 +420,46 @@ def backward_fused(view: CsrView, viewT: CsrView, perm: torch.Tensor, dY: torch.
     rc = lib.slk_backward_fused(ctypes.byref(view), ctypes.byref(viewT), ptr(perm), ptr(dY),
                                 ptr(X), dY.shape[1], ptr(dW), ptr(dbias), ptr(dX),
                                 stream_of(dY))
+    if rc:
+        _raise(rc)
+
+
+def quad_build(view: CsrView, perm: torch.Tensor | None, halves: int, device) -> QuadView:
+    """view's row quads (slk_quad_build) as a QuadView that holds its arrays; with
+    perm, for the values of the matrix that view's is the transpose of."""
+    lib = load()
+    nq = -(-view.nrows // 4)
+    nc = int(lib.slk_quad_chunks(view.ncols, halves))
+    n = int(lib.slk_quad_windows(ctypes.byref(view), halves))
+    words = nq * 4 * (nc + 1)
+    i32 = dict(dtype=torch.int32, device=device)
+    ws = torch.empty(words, **i32)
+    start, used = torch.empty(nc * nq, **i32), torch.empty(nq + 1, **i32)
+    count = torch.empty(nc * nq, dtype=torch.uint8, device=device)
+    offset, slot = torch.empty(64 * n, **i32), torch.empty(64 * n, **i32)
+    rc = lib.slk_quad_build(ctypes.byref(view), ptr(perm), halves, ptr(ws), words, ptr(start),
+                            ptr(count), ptr(offset), ptr(slot), n, ptr(used), stream_of(start))
+    if rc:
+        _raise(rc)
+    arrays = (start, count, offset, slot, used)
+    quads = QuadView(*(ptr(a) for a in arrays), n, halves)
+    quads.arrays = arrays
+    return quads
+
+
+def quad_halves(view: CsrView, N: int) -> int:
+    """Halves of the quads spmm_quad should run view with on N columns, 0 for
+    slk_spmm (slk_quad_halves)."""
+    return int(load().slk_quad_halves(ctypes.byref(view), N))
+
+
+def spmm_quad(view: CsrView, quads: QuadView, values: torch.Tensor, X: torch.Tensor,
+              Y: torch.Tensor, bias: torch.Tensor | None = None) -> None:
+    """Y = W·X (+ bias per row) through W's row quads (slk_spmm_quad), values
+    being what their slots index."""
+    ws = torch.empty(64 * quads.n_windows, dtype=torch.float32, device=Y.device)
+    rc = load().slk_spmm_quad(ctypes.byref(view), ctypes.byref(quads), ptr(values), ptr(ws), ptr(X),
+                              X.shape[0], X.shape[1], ptr(bias), ptr(Y), stream_of(Y))
     if rc:
         _raise(rc)
 

@@ -34,6 +34,10 @@ int64_t tuning(int knob);
 // Validates the parts of a CSR view every kernel relies on.
 int validate_csr(const slk_csr* W, const char* who);
 
+// Estimated microseconds of slk_spmm on W without schedules at N columns, for
+// callers that have another way to run it.
+double spmm_estimate(const slk_csr* W, int64_t N);
+
 // A second queue per device, for launchers that run two independent parts
 // of one call concurrently (slk_spmm's split forward, slk_sddmm's dense rows):
 // one stream (default priority) and the two events that fork it from and join

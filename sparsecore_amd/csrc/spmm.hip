@@ -1098,6 +1098,38 @@ double lds_cost(int64_t M, int64_t K, int64_t N, double density, int h, int rw) 
     return rounds * chunks * (40.0 + rw * (2.0 + density * kc * (h == 1 ? 4.0 : 6.0)));
 }
 
+// The LDS kernel's configuration for W at N columns (N a multiple of 4), *rw =
+// 0 if none qualifies; its lds_cost.
+double lds_choose(const slk_csr* W, int64_t N, int* h, int* rw) {
+    const int64_t M = W->nrows, K = W->ncols;
+    double best = 0.0;
+    *rw = 0;
+    if (N < kLdsMinN) return best;
+    const double density =
+        K > 0 ? static_cast<double>(W->total_capacity) / (1.2 * M * K) : 0.0;
+    // (3 and 6 rows per wave fit row counts such as 768 and 2304 to whole
+    // rounds of 256 workgroups: the 60M-GPT QKV input gradient, 768 rows,
+    // is 192 workgroups at 4 rows and 256 at 3)
+    for (const int cfg : {18, 16, 14, 13, 12, 28, 26, 24, 23, 22}) {  // h * 10 + rw
+        const int ch = cfg / 10, crw = cfg % 10;
+        // 8 rows x 8 columns per lane: rows of uniform length only (the
+        // light rows of a skewed matrix run slower with it: 16384^2
+        // Zipf(1.1) at 95%, forward as one split grid 6.97 -> 7.94 ms
+        // against 8 rows x 4 columns, while its transpose runs 6.91 ->
+        // 5.69 ms)
+        if (cfg == 28 && W->n_heavy_rows > 0) continue;
+        if (density * kLdsWaves * crw < kLdsMinReuse) continue;
+        if (lds_blocks(M, N, ch, crw) < kLdsMinBlocks) continue;
+        const double c = lds_cost(M, K, N, density, ch, crw);
+        if (*rw == 0 || c < best) {
+            best = c;
+            *rw = crw;
+            *h = ch;
+        }
+    }
+    return best;
+}
+
 // Y = W·X (+ bias per row): the shared body of slk_spmm and slk_spmm_bias.
 // Y^T for slk_spmm_t: one-row-per-wave kernel, one float per lane, each
 // lane writing its token's row of Yt (narrow layers; the stores of a wave are
@@ -1239,31 +1271,7 @@ int spmm_impl(const slk_csr* W, const float* X, int64_t K, int64_t N, const floa
     // SLK_TUNE_SPMM_KERNEL, SLK_TUNE_SPMM_H and SLK_TUNE_SPMM_RW override.
     const bool lds_ok = N % 4 == 0 && align % 16 == 0;
     int rw = 0, h = 1;
-    if (lds_ok && N >= kLdsMinN) {
-        const double density =
-            K > 0 ? static_cast<double>(W->total_capacity) / (1.2 * M * K) : 0.0;
-        double best = 0.0;
-        // (3 and 6 rows per wave fit row counts such as 768 and 2304 to whole
-        // rounds of 256 workgroups: the 60M-GPT QKV input gradient, 768 rows,
-        // is 192 workgroups at 4 rows and 256 at 3)
-        for (const int cfg : {18, 16, 14, 13, 12, 28, 26, 24, 23, 22}) {  // h * 10 + rw
-            const int ch = cfg / 10, crw = cfg % 10;
-            // 8 rows x 8 columns per lane: rows of uniform length only (the
-            // light rows of a skewed matrix run slower with it: 16384^2
-            // Zipf(1.1) at 95%, forward as one split grid 6.97 -> 7.94 ms
-            // against 8 rows x 4 columns, while its transpose runs 6.91 ->
-            // 5.69 ms)
-            if (cfg == 28 && W->n_heavy_rows > 0) continue;
-            if (density * kLdsWaves * crw < kLdsMinReuse) continue;
-            if (lds_blocks(M, N, ch, crw) < kLdsMinBlocks) continue;
-            const double c = lds_cost(M, K, N, density, ch, crw);
-            if (rw == 0 || c < best) {
-                best = c;
-                rw = crw;
-                h = ch;
-            }
-        }
-    }
+    if (lds_ok) lds_choose(W, N, &h, &rw);
     if (const int64_t t = tuning(SLK_TUNE_SPMM_KERNEL); t >= 0) {
         if (t == 0) rw = 0;
         if (t == 1 && lds_ok && rw == 0) rw = 8;
@@ -1337,6 +1345,23 @@ int spmm_impl(const slk_csr* W, const float* X, int64_t K, int64_t N, const floa
 }
 
 }  // namespace
+
+// Fitted like quad_cost, to the same 109 shapes: the LDS kernel 19.5 ns per
+// unit of lds_cost, the gather kernels the rate they reach once the slots
+// outweigh the launch (slots x columns per microsecond).
+double spmm_estimate(const slk_csr* W, int64_t N) {
+    const int64_t M = W->nrows;
+    if (N % 4 == 0) {
+        int h = 1, rw = 0;
+        const double c = lds_choose(W, N, &h, &rw);
+        if (rw != 0) return 4.0 + 0.0195 * c;
+    }
+    double rate = 3400.0;
+    if (N % 4 == 0 && M * ceil_div(N, 256) >= kTargetWaves) rate = 7200.0;
+    else if (N % 2 == 0 && M * ceil_div(N, 128) >= kTargetWaves) rate = 4200.0;
+    return 4.0 + W->total_capacity / 1.2 * N / (rate * 1e3);
+}
+
 }  // namespace slk
 
 extern "C" int slk_spmm(const slk_csr* W, const float* X, int64_t K, int64_t N, float* Y,

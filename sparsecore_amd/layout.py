@@ -294,6 +294,8 @@ class PaddedCSR:
         self._seglist = None    # key (topology_version, block_cols, seg_slots)
         self._phased = None     # key (topology_version, n_phases)
         self._binned = None     # key (topology_version, first, rw, h)
+        # (key (topology_version, halves, perm given), row quads)
+        self._quads_kept = None
         # True when a few columns hold many of the slots (a transpose of a
         # matrix with heavy rows): its gathers already stay in cache
         self._cols_skewed = False
@@ -503,6 +505,22 @@ class PaddedCSR:
             c = (key, base, view, c[3], c[4])
         self._binned = c
         return c[2]
+
+    def _quads(self, halves: int, perm: torch.Tensor | None = None) -> _lib.QuadView:
+        """The row quads of slk_spmm_quad for 64·halves columns a row, built on
+        the device (slk_quad_build, three launches, no host read) once per
+        topology. They list slots, not values, so they survive a change of
+        values. With perm (this matrix is a transpose, perm its slot map) the
+        slots are those of the matrix it was built from. Under graph capture the
+        build is only recorded, so its arrays are the graph's alone and not kept
+        for calls outside it."""
+        key = (self._topology_version, int(halves), perm is not None)
+        c = self._quads_kept
+        if c is None or c[0] != key:
+            c = (key, _lib.quad_build(self._view(), perm, int(halves), self.device))
+            if not torch.cuda.is_current_stream_capturing():
+                self._quads_kept = c
+        return c[1]
 
     def _rows_host(self):
         h = self._host_rows

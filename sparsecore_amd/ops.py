@@ -46,19 +46,26 @@ def _cached_transpose(W: PaddedCSR) -> PaddedCSR:
     Miss: rebuild on the device and store the entry. Entries are dropped when
     W is garbage collected, so a recycled id() can never return a stale WT.
     """
+    WT, perm, fresh = _transpose_entry(W)
+    if not fresh:
+        _lib.transpose_refresh(W.values, perm, WT.values)
+    return WT
+
+
+def _transpose_entry(W: PaddedCSR):
+    """(WT, perm, fresh) from the transpose cache, rebuilt when W's topology
+    changed; fresh: rebuilt by this call, with W's values."""
     key = id(W)
     cur_version = W.topology_version
     cur_shape = (int(W.nrows), int(W.ncols))
     cached = _transpose_cache.get(key)
     if cached is not None and cached[0] == cur_version and cached[1] == cur_shape:
-        _, _, WT, perm = cached
-        _lib.transpose_refresh(W.values, perm, WT.values)
-        return WT
+        return cached[2], cached[3], False
     WT, perm = transpose_with_perm(W)
     if cached is None:
         weakref.finalize(W, _drop_entry, key)
     _transpose_cache[key] = (cur_version, cur_shape, WT, perm)
-    return WT
+    return WT, perm, True
 
 
 def _rigl_update_cached(W: PaddedCSR, k_drop: int, dY: torch.Tensor, X: torch.Tensor) -> None:
@@ -93,13 +100,7 @@ def _cached_transpose_structure(W: PaddedCSR):
     (as ``_cached_transpose``) but without refreshing WT's values: for a
     caller that reads W's values through perm (slk_backward_fused). The next
     ``_cached_transpose`` refreshes them as on every hit."""
-    key = id(W)
-    cached = _transpose_cache.get(key)
-    if cached is not None and cached[0] == W.topology_version and \
-            cached[1] == (int(W.nrows), int(W.ncols)):
-        return cached[2], cached[3]
-    WT = _cached_transpose(W)
-    return WT, _transpose_cache[key][3]
+    return _transpose_entry(W)[:2]
 
 
 def _rebuild_stale_transposes(Ws) -> None:
@@ -187,8 +188,29 @@ def _bin_shape(W: PaddedCSR, K: int, N: int):
 # n column phases on slk_spmm's gather path (<= 1: none); "seg" = (block
 # columns, slots per segment) forces that segment list on slk_sddmm, () none;
 # "bin_shape" = (rows per wave, halves) forces that binned stream on
-# slk_spmm, False none.
+# slk_spmm, False none; "quad" = 1 or 2 forces row quads of that many halves,
+# 0 none.
 _overrides: dict[str, object] = {}
+
+
+# Row quads (slk_spmm_quad) instead of slk_spmm where slk_quad_halves expects
+# them to be faster: layers of some 5% density and up at N of about 1000 and up,
+# all but the smallest where N is not a multiple of 4 (2304 x 768, N = 8192,
+# 20%: 219 -> 169 us; 3072 x 768, N = 1001, 10%: 82 -> 35; 4096^2 x 4096, 10%:
+# 540 -> 398). Below _QUAD_MIN_WORK live slots x N no shape gains (the smallest
+# that does, 1152 x 384 at 10% and N = 1001, has 4.4e7), so the call is spared.
+_QUAD_MIN_WORK = 30_000_000
+
+
+def _quad_halves(W: PaddedCSR, K: int, N: int) -> int:
+    """64-column halves of the row quads (1 or 2) to run W on a K x N X with;
+    0: slk_spmm."""
+    forced = _overrides.get("quad")
+    if forced is not None:
+        return int(forced)
+    if W.nnz * N < _QUAD_MIN_WORK or "bin_shape" in _overrides or "spmm_phases" in _overrides:
+        return 0
+    return _lib.quad_halves(W._view(), N)
 
 
 def _spmm_view(W: PaddedCSR, X: torch.Tensor):
@@ -211,6 +233,10 @@ def _spmm_view(W: PaddedCSR, X: torch.Tensor):
 
 def _launch_spmm(W: PaddedCSR, X: torch.Tensor, bias: torch.Tensor | None = None) -> torch.Tensor:
     Y = torch.empty((W.nrows, X.shape[1]), dtype=torch.float32, device=X.device)
+    halves = _quad_halves(W, *X.shape)
+    if halves:
+        _lib.spmm_quad(W._view(), W._quads(halves), W.values, X, Y, bias)
+        return Y
     _lib.spmm(_spmm_view(W, X), X, Y, bias)
     return Y
 
@@ -352,8 +378,15 @@ def _spmm_backward(W: PaddedCSR, X: torch.Tensor, dY_f32: torch.Tensor, kernel: 
     if need_dw:
         dW_values = _launch_sddmm(W, dY_f32, _device_f32(X), kernel, dbias)
     if need_dx:
-        WT = _cached_transpose(W)
-        dX = _launch_spmm(WT, dY_f32)
+        WT, perm, fresh = _transpose_entry(W)
+        halves = _quad_halves(WT, *dY_f32.shape)
+        if halves:  # through W's values: no refresh of WT's
+            dX = torch.empty((W.ncols, dY_f32.shape[1]), dtype=torch.float32, device=W.device)
+            _lib.spmm_quad(WT._view(), WT._quads(halves, perm), W.values, dY_f32, dX)
+        else:
+            if not fresh:
+                _lib.transpose_refresh(W.values, perm, WT.values)
+            dX = _launch_spmm(WT, dY_f32)
     return dW_values, dX
 
 
