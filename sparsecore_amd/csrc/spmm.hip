@@ -1230,7 +1230,7 @@ int spmm_impl(const slk_csr* W, const float* X, int64_t K, int64_t N, const floa
             if (W->bin_first >= T) rest.bin_first = W->bin_first - T;
             else rest.bin_off = nullptr;  // a stream that covers dense rows is not used
         }
-        if (rest.nrows == 0) return SLK_OK;
+        if (rest.nrows == 0) return spmm_dense_rows(W, X, K, N, bias, Y, st);
         // With phase bounds (X far beyond the L2s), the dense rows run on the
         // caller's stream beside the phased gather of the light rows on the
         // side stream (the two-queue path below; the rest's heavy rows, if

@@ -35,7 +35,7 @@ import pytest
 import torch
 
 import oracle
-from helpers import from_oracle
+from helpers import assert_bits_equal, from_oracle
 from sparsecore_amd import _lib, layout, ops
 
 pytestmark = pytest.mark.gpu
@@ -347,3 +347,28 @@ def test_dense_rows_dw_refuses_an_n_it_cannot_take(dev):
         ops._overrides.update(old)
     np.testing.assert_array_equal(dW.cpu().numpy().view(np.uint32), want.view(np.uint32))
     del Xd
+
+
+@pytest.mark.parametrize("N", [70, 128])
+def test_every_row_dense(dev, N):
+    """A matrix of dense rows only: no rest beside them, forward and dW."""
+    M, K = 2048, 4096
+    rng = np.random.default_rng(N)
+    W = from_oracle(oracle.from_dense(
+        (rng.standard_normal((M, K)) * (rng.random((M, K)) < 0.3)).astype(np.float32)), dev)
+    assert W._view().n_dense_rows == M
+    X = torch.from_numpy(rng.standard_normal((K, N)).astype(np.float32)).to(dev)
+    dY = torch.from_numpy(rng.standard_normal((M, N)).astype(np.float32)).to(dev)
+    Y = torch.full((M, N), float("nan"), device=dev)
+    _lib.spmm(W._view(), X, Y)
+    ref = torch.empty_like(Y)
+    dW = ops._launch_sddmm(W, dY, X, "simd")
+    _lib.set_tuning("dense_rows", 0)
+    try:
+        _lib.spmm(W._view(), X, ref)
+    finally:
+        _lib.set_tuning("dense_rows", None)
+    _assert_equal_values(Y.cpu().numpy(), ref.cpu().numpy(), "Y")
+    want = torch.empty_like(dW)
+    _lib.sddmm(W._derived(W._view(), n_dense_rows=0), dY, X, want, _lib.SLK_DW_SIMD, None)
+    assert_bits_equal(dW.cpu().numpy(), want.cpu().numpy(), "dW")
