@@ -320,6 +320,47 @@ SLK_API int slk_sddmm_bias(const slk_csr* W, const float* dY, int64_t dY_rows,
                    const float* X, int64_t X_rows, int64_t N, float* dW,
                    float* dbias, int order, void* stream);
 
+/* A matrix's dW strips (slk_strip_build), the schedule of slk_sddmm_strips: one
+ * per topology. Rows at positions [first, nrows) of row_order (of the natural
+ * order with ordered = 0) are taken in quads; a strip is slots j·slots ..
+ * (j + 1)·slots - 1 of each row of a quad in one block of `block` columns (a
+ * multiple of 16 up to 256). items holds pairs {quad, block << 8 | j}, block by
+ * block (quad -1: padding to whole workgroups of 16 waves, per_wave strips
+ * each), rel, per quad, row and block, the first slot relative to row_start,
+ * used the number of workgroups. slots x per_wave: 48 x 1, 32 x 1, 16 x 1
+ * or 16 x 2, parts 1 or 2 (parts of 64 columns per staged window). */
+typedef struct slk_strips {
+    const int32_t* items;
+    const int32_t* rel;
+    const int32_t* used;
+    int64_t first;
+    int64_t ordered;
+    int64_t block;
+    int64_t slots;
+    int64_t per_wave;
+    int64_t parts;
+} slk_strips;
+
+/* Sizes (block, slots, per_wave, parts) with the least estimated time for dW of
+ * W at N columns, and that time in microseconds; block = 0 where slk_sddmm
+ * (estimated from W's capacity, shape and N) is about as fast or faster, or W
+ * has heavy or dense rows. Host only.                                       */
+SLK_API int slk_strip_choose(const slk_csr* W, int64_t N, slk_strips* T, double* us);
+/* words[0 .. 2]: int32 entries of items, rel and the build's scratch for W's
+ * strips of T's sizes.                                                      */
+SLK_API int slk_strip_words(const slk_csr* W, const slk_strips* T, int64_t* words);
+/* Builds them on the device: three launches, no host read. used: 1 word.     */
+SLK_API int slk_strip_build(const slk_csr* W, const slk_strips* T, int32_t* items, int32_t* rel,
+                    int32_t* used, int32_t* ws, void* stream);
+/* Bytes of slk_sddmm_strips' workspace: a copy of X, padded to 64 columns.   */
+SLK_API int64_t slk_strip_layout_bytes(int64_t ncols, int64_t N);
+/* slk_sddmm (SLK_DW_SIMD; with dbias slk_sddmm_bias) for W's strips, the same
+ * bits; slots of rows before `first` are left alone. N in [1, 2^21]. ws is
+ * scratch that the call overwrites.                                         */
+SLK_API int slk_sddmm_strips(const slk_csr* W, const slk_strips* T, const float* dY,
+                     const float* X, int64_t N, float* dW, float* dbias, void* ws,
+                     int64_t ws_bytes, void* stream);
+
 /* Transpose build, part 1 of 2 (replaces the index work of
  * `transpose_with_perm`, sparselab/layout.py:460-536).
  * Bytes of device workspace slk_transpose_count needs for W.                */

@@ -74,6 +74,11 @@ EXPORTS = (
     "slk_quad_halves",
     "slk_quad_build",
     "slk_spmm_quad",
+    "slk_strip_choose",
+    "slk_strip_words",
+    "slk_strip_build",
+    "slk_strip_layout_bytes",
+    "slk_sddmm_strips",
 )
 
 RIGL_INFO_BYTES = 32  # per row, slk_rigl_count's info
@@ -85,6 +90,8 @@ TUNE_KNOBS = {"spmm_kernel": 0, "spmm_h": 1, "spmm_rw": 2, "spmm_split": 3, "spm
               "sddmm_g": 5, "seg_lean": 6, "seg_group": 7, "transpose_tile": 8, "spmm_bin": 9,
               "spmm_g": 10, "rigl_tile": 11, "dense_rows": 12, "transpose_radix": 13,
               "quad_rw": 14}
+
+FORCED_KNOBS: set[str] = set()  # knobs that set_tuning holds off their automatic value
 
 BIN_MAX_CHUNKS = 960  # SLK_BIN_MAX_CHUNKS
 
@@ -145,6 +152,22 @@ class QuadView(ctypes.Structure):
     ]
 
 
+class StripView(ctypes.Structure):
+    """Mirror of ``slk_strips`` (include/sparsecore_amd.h)."""
+
+    _fields_ = [
+        ("items", ctypes.c_void_p),
+        ("rel", ctypes.c_void_p),
+        ("used", ctypes.c_void_p),
+        ("first", ctypes.c_int64),
+        ("ordered", ctypes.c_int64),
+        ("block", ctypes.c_int64),
+        ("slots", ctypes.c_int64),
+        ("per_wave", ctypes.c_int64),
+        ("parts", ctypes.c_int64),
+    ]
+
+
 _lib = None
 _load_error: str | None = None
 
@@ -197,6 +220,13 @@ def _declare(lib) -> None:
     lib.slk_quad_build.argtypes = [_csrp, _vp, _i64, _vp, _i64, _vp, _vp, _vp, _vp, _i64, _vp, _vp]
     lib.slk_spmm_quad.argtypes = [_csrp, ctypes.POINTER(QuadView), _vp, _vp, _vp, _i64, _i64, _vp,
                                   _vp, _vp]
+    stripp = ctypes.POINTER(StripView)
+    lib.slk_strip_choose.argtypes = [_csrp, _i64, stripp, ctypes.POINTER(ctypes.c_double)]
+    lib.slk_strip_words.argtypes = [_csrp, stripp, ctypes.POINTER(_i64)]
+    lib.slk_strip_build.argtypes = [_csrp, stripp, _vp, _vp, _vp, _vp, _vp]
+    lib.slk_strip_layout_bytes.restype = _i64
+    lib.slk_strip_layout_bytes.argtypes = [_i64, _i64]
+    lib.slk_sddmm_strips.argtypes = [_csrp, stripp, _vp, _vp, _i64, _vp, _vp, _vp, _i64, _vp]
     lib.slk_phase_bounds_build.argtypes = [_csrp, _i64, _vp, _vp]
     lib.slk_set_tuning.argtypes = [ctypes.c_int, _i64]
     lib.slk_rigl_norms.argtypes = [_vp, _i64, _vp, _i64, _i64, _vp, _vp, _vp]
@@ -221,7 +251,7 @@ def _declare(lib) -> None:
              "slk_drop_grow_workspace_bytes", "slk_rigl_bound_factor", "slk_rigl_partial_factor",
              "slk_dense_grad_approx_workspace_bytes",
              "slk_seg_list_capacity", "slk_seg_list_workspace_bytes", "slk_quad_windows",
-             "slk_quad_chunks", "slk_quad_halves")
+             "slk_quad_chunks", "slk_quad_halves", "slk_strip_layout_bytes")
     for name in EXPORTS:
         if name not in sized:
             getattr(lib, name).restype = ctypes.c_int
@@ -464,6 +494,48 @@ def spmm_quad(view: CsrView, quads: QuadView, values: torch.Tensor, X: torch.Ten
         _raise(rc)
 
 
+def strip_choose(view: CsrView, N: int) -> tuple[tuple[int, int, int, int] | None, float]:
+    """((block, slots, per_wave, parts), estimated us) of the dW strips for view
+    at N columns; (None, 0.0) if there are none (slk_strip_choose)."""
+    T, us = StripView(), ctypes.c_double()
+    rc = load().slk_strip_choose(ctypes.byref(view), N, ctypes.byref(T), ctypes.byref(us))
+    if rc:
+        _raise(rc)
+    return ((T.block, T.slots, T.per_wave, T.parts) if T.block else None), us.value
+
+
+def strip_build(view: CsrView, first: int, ordered: bool, block: int, slots: int, per_wave: int,
+                parts: int, device) -> StripView:
+    """view's dW strips (slk_strip_build) as a StripView that holds its arrays."""
+    lib = load()
+    T = StripView(None, None, None, first, int(ordered), block, slots, per_wave, parts)
+    words = (ctypes.c_int64 * 3)()
+    rc = lib.slk_strip_words(ctypes.byref(view), ctypes.byref(T), words)
+    if rc:
+        _raise(rc)
+    items, rel, ws = (torch.empty(n, dtype=torch.int32, device=device) for n in words)
+    used = torch.empty(1, dtype=torch.int32, device=device)
+    rc = lib.slk_strip_build(ctypes.byref(view), ctypes.byref(T), ptr(items), ptr(rel), ptr(used),
+                             ptr(ws), stream_of(items))
+    if rc:
+        _raise(rc)
+    T.items, T.rel, T.used = ptr(items), ptr(rel), ptr(used)
+    T.arrays = (items, rel, used)
+    return T
+
+
+def sddmm_strips(view: CsrView, strips: StripView, dY: torch.Tensor, X: torch.Tensor,
+                 dW: torch.Tensor, dbias: torch.Tensor | None = None) -> None:
+    """dW in the SIMD order (and dbias) of the strips' rows (slk_sddmm_strips)."""
+    lib = load()
+    nbytes = int(lib.slk_strip_layout_bytes(view.ncols, X.shape[1]))
+    ws = torch.empty(nbytes, dtype=torch.uint8, device=dW.device)
+    rc = lib.slk_sddmm_strips(ctypes.byref(view), ctypes.byref(strips), ptr(dY), ptr(X),
+                              X.shape[1], ptr(dW), ptr(dbias), ptr(ws), nbytes, stream_of(dW))
+    if rc:
+        _raise(rc)
+
+
 def seg_list_build(view: CsrView, block_cols: int, seg_slots: int, device):
     """(seg_start, seg_row, seg_count, seg_groups) int32 tensors: W's live slots
     cut into segments of at most seg_slots slots of one row inside one column
@@ -578,6 +650,10 @@ def set_tuning(knob: str, value: int | None) -> None:
     rc = load().slk_set_tuning(TUNE_KNOBS[knob], -1 if value is None else int(value))
     if rc:
         _raise(rc)
+    if value is None or int(value) < 0:
+        FORCED_KNOBS.discard(knob)
+    else:
+        FORCED_KNOBS.add(knob)
 
 
 def rigl_norms(dY: torch.Tensor, X: torch.Tensor, nrm_dY: torch.Tensor,

@@ -80,10 +80,31 @@ __device__ __forceinline__ void bias_row_sum(const float* __restrict__ dY, int64
     const int lane = threadIdx.x & (kWave - 1);
     const float* p = dY + row * rs;
     float acc = 0.0f;
-    for (int64_t j = lane; j < N; j += kWave) acc = acc + p[j * js];
+    int64_t j = lane;
+    for (; j + 7 * kWave < N; j += 8 * kWave) {  // eight loads in flight, added in order
+        float v[8];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) v[i] = p[(j + i * kWave) * js];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) acc = acc + v[i];
+    }
+    for (; j < N; j += kWave) acc = acc + p[j * js];
 #pragma unroll
     for (int off = kWave / 2; off > 0; off >>= 1) acc = acc + __shfl_xor(acc, off);
     if (lane == 0) dbias[row] = acc;
+}
+
+// Zeroes the padding slots of one row of dW (one wave): used where the slots
+// are walked through a schedule that lists live slots only.
+__device__ __forceinline__ void zero_row_padding(const int32_t* __restrict__ row_start,
+                                                 const int32_t* __restrict__ row_nnz,
+                                                 const int32_t* __restrict__ row_cap, int64_t M,
+                                                 int64_t row, float* __restrict__ dW) {
+    if (row >= M) return;
+    const int lane = threadIdx.x & (kWave - 1);
+    const int64_t s0 = row_start[row];
+    const int64_t e = s0 + row_cap[row];
+    for (int64_t s = s0 + row_nnz[row] + lane; s < e; s += kWave) dW[s] = 0.0f;
 }
 
 }  // namespace slk

@@ -255,19 +255,6 @@ __device__ __forceinline__ void wave_sync() {
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-// Zeroes the padding slots of one row of dW (one wave): used where the slots
-// are walked through a schedule that lists live slots only.
-__device__ __forceinline__ void zero_row_padding(const int32_t* __restrict__ row_start,
-                                                 const int32_t* __restrict__ row_nnz,
-                                                 const int32_t* __restrict__ row_cap, int64_t M,
-                                                 int64_t row, float* __restrict__ dW) {
-    if (row >= M) return;
-    const int lane = threadIdx.x & (kWave - 1);
-    const int64_t s0 = row_start[row];
-    const int64_t e = s0 + row_cap[row];
-    for (int64_t s = s0 + row_nnz[row] + lane; s < e; s += kWave) dW[s] = 0.0f;
-}
-
 template <int G>
 __global__ __launch_bounds__(kBlock) void sddmm_simd_win_kernel(
     int64_t M, int64_t N, int64_t cap_total,

@@ -294,8 +294,10 @@ class PaddedCSR:
         self._seglist = None    # key (topology_version, block_cols, seg_slots)
         self._phased = None     # key (topology_version, n_phases)
         self._binned = None     # key (topology_version, first, rw, h)
-        # (key (topology_version, halves, perm given), row quads)
-        self._quads_kept = None
+        # topology_version, then schedules by key: at most _KEEP each
+        self._quads_kept = (-1, {})   # (halves, perm given): row quads
+        self._strips_kept = (-1, {})  # (block, slots, per_wave, parts): dW strips
+        self._strip_sizes = (-1, {})  # N: the strips' sizes, or None
         # True when a few columns hold many of the slots (a transpose of a
         # matrix with heavy rows): its gathers already stay in cache
         self._cols_skewed = False
@@ -514,13 +516,39 @@ class PaddedCSR:
         slots are those of the matrix it was built from. Under graph capture the
         build is only recorded, so its arrays are the graph's alone and not kept
         for calls outside it."""
-        key = (self._topology_version, int(halves), perm is not None)
-        c = self._quads_kept
-        if c is None or c[0] != key:
-            c = (key, _lib.quad_build(self._view(), perm, int(halves), self.device))
-            if not torch.cuda.is_current_stream_capturing():
-                self._quads_kept = c
-        return c[1]
+        return self._kept("_quads_kept", (int(halves), perm is not None),
+                          lambda: _lib.quad_build(self._view(), perm, int(halves), self.device))
+
+    # Schedules of one kind kept per topology: sizes follow N, so a program that
+    # alternates between a few N (training and evaluation batches) builds each once.
+    _KEEP = 4
+
+    def _kept(self, name: str, key, build):
+        version, kept = getattr(self, name)
+        if version != self._topology_version:
+            kept = {}
+            setattr(self, name, (self._topology_version, kept))
+        if key in kept:
+            return kept[key]
+        value = build()
+        if not torch.cuda.is_current_stream_capturing():
+            while len(kept) >= self._KEEP:
+                kept.pop(next(iter(kept)), None)
+            kept[key] = value
+        return value
+
+    def _strips(self, sizes) -> _lib.StripView:
+        """The dW strips of slk_sddmm_strips for sizes (block, slots, per_wave,
+        parts), built on the device (slk_strip_build, three launches, no host
+        read) and kept like the quads."""
+        return self._kept("_strips_kept", tuple(sizes),
+                          lambda: _lib.strip_build(self._view(), 0, False, *sizes, self.device))
+
+    def _strip_choice(self, N: int):
+        """Sizes of the strips that dW should run with at N columns, None for
+        slk_sddmm (slk_strip_choose; host arithmetic of some 10 us, so kept)."""
+        return self._kept("_strip_sizes", int(N),
+                          lambda: _lib.strip_choose(self._view(), int(N))[0])
 
     def _rows_host(self):
         h = self._host_rows

@@ -189,7 +189,8 @@ def _bin_shape(W: PaddedCSR, K: int, N: int):
 # columns, slots per segment) forces that segment list on slk_sddmm, () none;
 # "bin_shape" = (rows per wave, halves) forces that binned stream on
 # slk_spmm, False none; "quad" = 1 or 2 forces row quads of that many halves,
-# 0 none.
+# 0 none; "strips" = (block, slots, per_wave, parts) forces those strips for dW,
+# None none.
 _overrides: dict[str, object] = {}
 
 
@@ -291,10 +292,34 @@ def _sddmm_view(W: PaddedCSR, X: torch.Tensor):
     return W._view()
 
 
+# Strips (slk_sddmm_strips) instead of slk_sddmm where slk_strip_choose expects
+# them to be faster: N not a multiple of 4 (1537 x 1000 at 20%, N = 1777: 194 ->
+# 56 us), N below 1024 or too few slots for the segment list (512 x 784 at 20%, N
+# = 8192: 159 -> 108), and layers around 3-5% and 20-40% (4096^2 x 4096 at 5%: 585
+# -> 380; 2304 x 768 at 30%, N = 8192: 373 -> 280). Below _STRIP_MIN_WORK live
+# slots x N no shape gains.
+_STRIP_MIN_WORK = 30_000_000
+
+
+def _strip_sizes(W: PaddedCSR, N: int):
+    """(block, slots, per_wave, parts) of the strips to run W's dW with at N
+    columns; None: slk_sddmm."""
+    if "strips" in _overrides:
+        return _overrides["strips"]
+    if W.nnz * N < _STRIP_MIN_WORK or "seg" in _overrides or "dense_dw" in _overrides or \
+            not _lib.FORCED_KNOBS.isdisjoint(("sddmm_g", "seg_lean", "seg_group")):
+        return None
+    return W._strip_choice(N)
+
+
 def _launch_sddmm(W: PaddedCSR, dY: torch.Tensor, X: torch.Tensor, kernel: str,
                   dbias: torch.Tensor | None = None) -> torch.Tensor:
     dW = torch.empty(W.total_capacity, dtype=torch.float32, device=X.device)
     order = _lib.SLK_DW_SCALAR if kernel == "scalar" else _lib.SLK_DW_SIMD
+    sizes = _strip_sizes(W, X.shape[1]) if order == _lib.SLK_DW_SIMD else None
+    if sizes:
+        _lib.sddmm_strips(W._view(), W._strips(sizes), dY, X, dW, dbias)
+        return dW
     view = _sddmm_view(W, X) if order == _lib.SLK_DW_SIMD else W._view()
     _lib.sddmm(view, dY, X, dW, order, dbias)
     return dW
