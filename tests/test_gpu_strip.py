@@ -131,3 +131,31 @@ def test_default_route_takes_strips_and_follows_the_topology(dev):
         _lib.sddmm(W._view(), dY, X, want, _lib.SLK_DW_SIMD, None)
         assert_bits_equal(dW.cpu().numpy(), want.cpu().numpy(), f"dW, step {step}")
         W.rewrite_row(3, list(range(0, 200, 2)), [1.0] * 100)
+
+
+def test_strips_built_under_capture_stay_with_the_graph(dev, monkeypatch):
+    """A first dW under graph capture records choice, build and launch; replays,
+    with eager work between them, give the eager bits, and the matrix keeps no
+    arrays that only the graph fills."""
+    monkeypatch.setitem(ops._overrides, "strips", (144, 48, 1, 2))  # over 64 KiB of LDS
+    c = _mixed(200, 300, seed=11)
+    W = from_oracle(c, dev)
+    rng = np.random.default_rng(12)
+    X = _t(rng.standard_normal((300, 129)).astype(np.float32), dev)
+    dY = _t(rng.standard_normal((200, 129)).astype(np.float32), dev)
+    W._view()
+    stream = torch.cuda.Stream()
+    stream.wait_stream(torch.cuda.current_stream())
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.stream(stream):
+        ops._launch_sddmm(from_oracle(c, dev), dY, X, "simd")  # warm-up on another matrix
+        with torch.cuda.graph(graph, stream=stream):
+            dW = ops._launch_sddmm(W, dY, X, "simd")
+    torch.cuda.current_stream().wait_stream(stream)
+    assert not W._strips_kept[1]
+    for step in range(3):
+        dY.mul_(1.5)
+        graph.replay()
+        torch.cuda.synchronize()
+        assert_bits_equal(dW.cpu().numpy(), ops._launch_sddmm(W, dY, X, "simd").cpu().numpy(),
+                          f"replay {step}")
