@@ -296,7 +296,13 @@ def _raise(rc: int) -> None:
 
 
 def stream_of(t: torch.Tensor) -> int:
-    return torch.cuda.current_stream(t.device).cuda_stream
+    """The raw current stream of t's device, read on every call. Not through
+    torch.cuda.current_stream, which builds a Stream object each time: a small
+    layer's pass is bound by such host work around its launches."""
+    device = t.device
+    if device.type != "cuda":
+        return torch.cuda.current_stream(device).cuda_stream  # raises as it did
+    return torch._C._cuda_getCurrentRawStream(device.index)
 
 
 def ptr(t: torch.Tensor | None) -> int | None:
