@@ -185,6 +185,30 @@ def _check_host(nrows, ncols, values, col, rs, nnz, cap) -> str:
 #  PaddedCSR
 # ─────────────────────────────────────────────────────────────────────
 
+class _Built:
+    """Device arrays that a lazy build has queued on the current stream, kept
+    for later calls on any stream: `event` is recorded behind the build."""
+
+    __slots__ = ("value", "arrays", "stream", "event")
+
+    def __init__(self, value, arrays):
+        stream = torch.cuda.current_stream(arrays[0].device)
+        self.value, self.arrays, self.stream = value, arrays, stream.cuda_stream
+        # (what a capture builds is not kept, so nothing waits for it)
+        self.event = None if torch.cuda.is_current_stream_capturing() else stream.record_event()
+
+    def join(self) -> None:
+        """Orders the current stream behind the build. The allocator is told of
+        a stream other than the build's, so that arrays dropped by their matrix
+        are not given away while that stream still reads them."""
+        if _lib.stream_of(self.arrays[0]) == self.stream:
+            return
+        stream = torch.cuda.current_stream(self.arrays[0].device)
+        stream.wait_event(self.event)
+        for a in self.arrays:
+            a.record_stream(stream)
+
+
 # A row is "heavy" for slk_spmm's LDS-staged kernel when it holds more than
 # this many times the mean row's slots (slk_csr.n_heavy_rows). Measured on the
 # 16384^2 Zipf(1.1) layer at 95% sparsity, with heavy rows at 8 columns per
@@ -289,15 +313,21 @@ class PaddedCSR:
         self._nnz = nnz
         self._topology_version = 0
         self._cview = None
-        self._order = None      # (topology_version, device row schedule, heavy rows)
-        # derived views: (key, the base view they copy, view, schedule arrays)
-        self._seglist = None    # key (topology_version, block_cols, seg_slots)
-        self._phased = None     # key (topology_version, n_phases)
-        self._binned = None     # key (topology_version, first, rw, h)
-        # topology_version, then schedules by key: at most _KEEP each
+        # (topology_version, row order, heavy rows, dense rows, dense scratch, _Built)
+        self._order = None
+        # schedules: topology_version, then by key a _Built (see _kept)
+        self._segs_kept = (-1, {})    # (block_cols, seg_slots, dense rows left out)
+        self._phases_kept = (-1, {})  # n_phases
+        self._bins_kept = (-1, {})    # (first, rw, h)
         self._quads_kept = (-1, {})   # (halves, perm given): row quads
         self._strips_kept = (-1, {})  # (block, slots, per_wave, parts): dW strips
-        self._strip_sizes = (-1, {})  # N: the strips' sizes, or None
+        # the last derived view of a kind: (key, the base view it copies, view, arrays)
+        self._seglist = None
+        self._phased = None
+        self._binned = None
+        self._strip_sizes = (-1, {})  # topology_version, N: the strips' sizes, or None
+        # topology_version and what graphs captured under it read (see _pin)
+        self._pinned = (-1, [])
         # True when a few columns hold many of the slots (a transpose of a
         # matrix with heavy rows): its gathers already stay in cache
         self._cols_skewed = False
@@ -391,9 +421,10 @@ class PaddedCSR:
     def _view(self) -> _lib.CsrView:
         v = self._cview
         if v is None:
-            order, n_heavy, n_dense, dws = None, 0, 0, None
+            order, n_heavy, n_dense, dws, built = None, 0, 0, None, None
             if self._nrows >= self._ORDER_MIN_ROWS and self._on_device():
-                if self._order is None or self._order[0] != self._topology_version:
+                c = self._order
+                if c is None or c[0] != self._topology_version:
                     # stable: equal-length rows keep their natural order
                     heavy, dense = self._heavy_hint, self._dense_hint
                     if heavy is None or dense is None:
@@ -402,27 +433,89 @@ class PaddedCSR:
                             heavy = heavy_row_count(nz)
                         if dense is None:
                             dense = dense_row_count(nz, self._ncols)
-                    ws = None
-                    if dense:
-                        ws = torch.empty(_lib.dense_rows_workspace_bytes(dense, self._ncols),
-                                         dtype=torch.uint8, device=self._values.device)
-                    self._order = (self._topology_version,
-                                   torch.argsort(self._row_nnz, descending=True,
-                                                 stable=True).to(_I32), heavy, dense, ws)
-                order, n_heavy, n_dense, dws = self._order[1:5]
+                    order = torch.argsort(self._row_nnz, descending=True, stable=True).to(_I32)
+                    dws = self._dense_scratch(dense)
+                    arrays = (order,) if dws is None else (order, dws)
+                    c = (self._topology_version, order, heavy, dense, dws, _Built(None, arrays))
+                    if not torch.cuda.is_current_stream_capturing():
+                        self._order = c
+                order, n_heavy, n_dense, dws, built = c[1:6]
             v = _lib.CsrView(self._nrows, self._ncols, self._values.numel(),
                              _lib.ptr(self._values), _lib.ptr(self._col), _lib.ptr(self._rs),
                              _lib.ptr(self._row_nnz), _lib.ptr(self._row_cap), _lib.ptr(order),
                              n_heavy_rows=n_heavy, n_dense_rows=n_dense,
                              dense_ws=_lib.ptr(dws))
+            v.built = built
+            if built is not None and torch.cuda.is_current_stream_capturing():
+                # an order that only the graph fills is the graph's alone
+                if self._order is None or self._order[5] is not built:
+                    return v
             self._cview = v
+        built = v.built
+        if built is None:
+            return v
+        if torch.cuda.is_current_stream_capturing():
+            self._pin(built)
+        elif _lib.stream_of(self._col) == built.stream:
+            return v
+        else:
+            built.join()
+        if v.n_dense_rows:  # the kept scratch belongs to calls on the build's stream
+            own = self._dense_scratch(v.n_dense_rows)
+            v = self._derived(v, dense_ws=_lib.ptr(own))
+            v.own = own
         return v
+
+    def _dense_scratch(self, n_dense: int) -> torch.Tensor | None:
+        """Scratch of the matrix-core path for n_dense dense rows; None for 0."""
+        if not n_dense:
+            return None
+        return torch.empty(_lib.dense_rows_workspace_bytes(n_dense, self._ncols),
+                           dtype=torch.uint8, device=self._values.device)
 
     @staticmethod
     def _derived(base: _lib.CsrView, **changes) -> _lib.CsrView:
         fields = {f: getattr(base, f) for f, _ in _lib.CsrView._fields_}
         fields.update(changes)
-        return _lib.CsrView(**fields)
+        v = _lib.CsrView(**fields)
+        v.base = base  # and with it the arrays that only the base holds
+        return v
+
+    # Lazily built device state (row order, schedules) is kept per topology. A
+    # call on another stream than the build's waits for the build (_Built.join).
+    # A graph captured on kept arrays holds their addresses, so they are pinned:
+    # they outlive a change of the topology until a capture under a newer one.
+    # What is first built under capture is the graph's alone and not kept, since
+    # only replays fill it.
+
+    def _pin(self, held) -> None:
+        version, pinned = self._pinned
+        if version != self._topology_version:
+            pinned = []
+            self._pinned = (self._topology_version, pinned)
+        if not any(p is held for p in pinned):
+            pinned.append(held)
+
+    def _kept(self, name: str, key, build, recorded: bool = False):
+        """build()'s (value, arrays), kept under `key` for this topology; the
+        value. recorded: under capture always build anew, into the graph, whose
+        replays then follow the matrix's rows as they are."""
+        version, kept = getattr(self, name)
+        if version != self._topology_version:
+            kept = {}
+            setattr(self, name, (self._topology_version, kept))
+        capturing = torch.cuda.is_current_stream_capturing()
+        b = None if capturing and recorded else kept.get(key)
+        if b is None:
+            value, arrays = build()
+            if not capturing:
+                kept[key] = _Built(value, arrays)
+            return value
+        if capturing:
+            self._pin(b)
+        else:
+            b.join()
+        return b.value
 
     def _view_segmented(self, block_cols: int, seg_slots: int,
                         skip_dense: bool = False) -> _lib.CsrView:
@@ -438,20 +531,22 @@ class PaddedCSR:
         topology does."""
         base = self._view()
         skip = int(base.n_dense_rows) if skip_dense else 0
-        key = (self._topology_version, int(block_cols), int(seg_slots), skip)
+        key = (int(block_cols), int(seg_slots), skip)
+
+        def build():
+            arrays = _lib.seg_list_build(self._derived(base, seg_dense_rows=skip), key[0], key[1],
+                                         self.device)
+            return arrays, arrays
+
+        arrays = self._kept("_segs_kept", key, build)
         c = self._seglist
-        if c is None or c[0] != key:
-            arrays = _lib.seg_list_build(self._derived(base, seg_dense_rows=skip), int(block_cols),
-                                         int(seg_slots), self.device)
-            c = (key, None, None, arrays)
-        if c[1] is not base:
-            start, row, count, groups = c[3]
+        if c is None or c[1] is not base or c[3] is not arrays:
+            start, row, count, groups = arrays
             view = self._derived(base, seg_start=_lib.ptr(start), seg_row=_lib.ptr(row),
                                  seg_count=_lib.ptr(count), seg_groups=_lib.ptr(groups),
-                                 n_seg=int(start.numel()), seg_block=int(block_cols),
-                                 seg_slots=int(seg_slots), seg_dense_rows=skip)
-            c = (key, base, view, c[3])
-        self._seglist = c
+                                 n_seg=int(start.numel()), seg_block=key[0], seg_slots=key[1],
+                                 seg_dense_rows=skip)
+            c = self._seglist = (key, base, view, arrays)
         return c[2]
 
     def _view_phased(self, n_phases: int) -> _lib.CsrView:
@@ -461,14 +556,17 @@ class PaddedCSR:
         Built on the device (slk_phase_bounds_build, one launch) once per
         topology; the cached view follows the base view as above."""
         base = self._view()
-        key = (self._topology_version, int(n_phases))
+        key = int(n_phases)
+
+        def build():
+            lo = _lib.phase_bounds_build(base, key, self.device)
+            return lo, (lo,)
+
+        lo = self._kept("_phases_kept", key, build)
         c = self._phased
-        if c is None or c[0] != key:
-            c = (key, None, None, _lib.phase_bounds_build(base, int(n_phases), self.device))
-        if c[1] is not base:
-            view = self._derived(base, phase_lo=_lib.ptr(c[3]), n_phases=int(n_phases))
-            c = (key, base, view, c[3])
-        self._phased = c
+        if c is None or c[1] is not base or c[3] is not lo:
+            view = self._derived(base, phase_lo=_lib.ptr(lo), n_phases=key)
+            c = self._phased = (key, base, view, lo)
         return c[2]
 
     def _bin_coverage(self) -> tuple[int, int]:
@@ -493,19 +591,21 @@ class PaddedCSR:
         launches, no host read) once per topology; the cached view follows the
         base view as the other schedules do."""
         base = self._view()
-        first, n_bin = self._bin_coverage()
-        key = (self._topology_version, first, int(rw), int(h))
+
+        def build():
+            first, n_bin = self._bin_coverage()
+            arrays = _lib.bin_build(base, first, int(rw), int(h), n_bin, self.device)
+            return (first, n_bin, arrays), arrays
+
+        kept = self._kept("_bins_kept", (int(base.n_heavy_rows), int(rw), int(h)), build)
         c = self._binned
-        if c is None or c[0] != key:
-            c = (key, None, None,
-                 _lib.bin_build(base, first, int(rw), int(h), n_bin, self.device), n_bin)
-        if c[1] is not base:
-            off, slot, cnt, start = c[3]
+        if c is None or c[1] is not base or c[3] is not kept[2]:
+            first, n_bin, arrays = kept
+            off, slot, cnt, start = arrays
             view = self._derived(base, bin_off=_lib.ptr(off), bin_slot=_lib.ptr(slot),
                                  bin_cnt=_lib.ptr(cnt), bin_start=_lib.ptr(start),
-                                 bin_first=first, bin_rw=int(rw), bin_h=int(h), n_bin=c[4])
-            c = (key, base, view, c[3], c[4])
-        self._binned = c
+                                 bin_first=first, bin_rw=int(rw), bin_h=int(h), n_bin=n_bin)
+            c = self._binned = ((first, int(rw), int(h)), base, view, arrays)
         return c[2]
 
     def _quads(self, halves: int, perm: torch.Tensor | None = None) -> _lib.QuadView:
@@ -514,41 +614,39 @@ class PaddedCSR:
         topology. They list slots, not values, so they survive a change of
         values. With perm (this matrix is a transpose, perm its slot map) the
         slots are those of the matrix it was built from. Under graph capture the
-        build is only recorded, so its arrays are the graph's alone and not kept
-        for calls outside it."""
-        return self._kept("_quads_kept", (int(halves), perm is not None),
-                          lambda: _lib.quad_build(self._view(), perm, int(halves), self.device))
+        build is recorded with the call, so that a replay follows the rows as
+        they are."""
+        def build():
+            q = _lib.quad_build(self._view(), perm, int(halves), self.device)
+            return q, q.arrays
 
-    # Schedules of one kind kept per topology: sizes follow N, so a program that
-    # alternates between a few N (training and evaluation batches) builds each once.
-    _KEEP = 4
-
-    def _kept(self, name: str, key, build):
-        version, kept = getattr(self, name)
-        if version != self._topology_version:
-            kept = {}
-            setattr(self, name, (self._topology_version, kept))
-        if key in kept:
-            return kept[key]
-        value = build()
-        if not torch.cuda.is_current_stream_capturing():
-            while len(kept) >= self._KEEP:
-                kept.pop(next(iter(kept)), None)
-            kept[key] = value
-        return value
+        return self._kept("_quads_kept", (int(halves), perm is not None), build, recorded=True)
 
     def _strips(self, sizes) -> _lib.StripView:
         """The dW strips of slk_sddmm_strips for sizes (block, slots, per_wave,
         parts), built on the device (slk_strip_build, three launches, no host
-        read) and kept like the quads."""
-        return self._kept("_strips_kept", tuple(sizes),
-                          lambda: _lib.strip_build(self._view(), 0, False, *sizes, self.device))
+        read) and kept, or recorded, like the quads."""
+        def build():
+            t = _lib.strip_build(self._view(), 0, False, *sizes, self.device)
+            return t, t.arrays
+
+        return self._kept("_strips_kept", tuple(sizes), build, recorded=True)
+
+    # Strip choices kept per topology, by N.
+    _KEEP = 4
 
     def _strip_choice(self, N: int):
         """Sizes of the strips that dW should run with at N columns, None for
         slk_sddmm (slk_strip_choose; host arithmetic of some 10 us, so kept)."""
-        return self._kept("_strip_sizes", int(N),
-                          lambda: _lib.strip_choose(self._view(), int(N))[0])
+        version, kept = self._strip_sizes
+        if version != self._topology_version:
+            kept = {}
+            self._strip_sizes = (self._topology_version, kept)
+        if N not in kept:
+            while len(kept) >= self._KEEP:
+                kept.pop(next(iter(kept)), None)
+            kept[N] = _lib.strip_choose(self._view(), int(N))[0]
+        return kept[N]
 
     def _rows_host(self):
         h = self._host_rows

@@ -60,6 +60,8 @@ def _transpose_entry(W: PaddedCSR):
     cur_shape = (int(W.nrows), int(W.ncols))
     cached = _transpose_cache.get(key)
     if cached is not None and cached[0] == cur_version and cached[1] == cur_shape:
+        if torch.cuda.is_current_stream_capturing():
+            W._pin(cached)  # the graph reads WT's arrays and perm
         return cached[2], cached[3], False
     WT, perm = transpose_with_perm(W)
     if cached is None:
@@ -202,6 +204,24 @@ _overrides: dict[str, object] = {}
 # that does, 1152 x 384 at 10% and N = 1001, has 4.4e7), so the call is spared.
 _QUAD_MIN_WORK = 30_000_000
 
+# Under graph capture a call records the build of its quads or strips with
+# itself, so that a replay follows the rows as they are and the graph owns all
+# that it reads. The build adds 9-20 us to each replay (4096 x 1024 to 4096^2 at
+# 30% the most), which they repay from this many live slots x N on: where N is
+# not a multiple of 4 (1152 x 384 at 30%, N = 1001: forward 49 -> 44 us, dW 42 ->
+# 40; 2304 x 768 at 30%, N = 1001: 161 -> 74, 145 -> 65; 4096 x 1024 at 10%, N =
+# 333, below the line: dW 53 -> 57) and where it is (2304 x 768 at 30%, N = 8192:
+# 289 -> 269, 367 -> 300; 3072 x 768 at 30%, N = 2048, below: 107 -> 109).
+_CAPTURED_MIN_WORK = 200_000_000
+_CAPTURED_MIN_WORK_ALIGNED = 3_000_000_000
+
+
+def _recording_pays(W: PaddedCSR, N: int) -> bool:
+    """False where this call is captured and the build of quads or strips, run
+    by every replay, would cost more than they gain."""
+    return not torch.cuda.is_current_stream_capturing() or \
+        W.nnz * N >= (_CAPTURED_MIN_WORK if N % 4 else _CAPTURED_MIN_WORK_ALIGNED)
+
 
 def _quad_halves(W: PaddedCSR, K: int, N: int) -> int:
     """64-column halves of the row quads (1 or 2) to run W on a K x N X with;
@@ -211,7 +231,8 @@ def _quad_halves(W: PaddedCSR, K: int, N: int) -> int:
         return int(forced)
     if W.nnz * N < _QUAD_MIN_WORK or "bin_shape" in _overrides or "spmm_phases" in _overrides:
         return 0
-    return _lib.quad_halves(W._view(), N)
+    halves = _lib.quad_halves(W._view(), N)
+    return halves if halves and _recording_pays(W, N) else 0
 
 
 def _spmm_view(W: PaddedCSR, X: torch.Tensor):
@@ -232,9 +253,12 @@ def _spmm_view(W: PaddedCSR, X: torch.Tensor):
     return W._view()
 
 
-def _launch_spmm(W: PaddedCSR, X: torch.Tensor, bias: torch.Tensor | None = None) -> torch.Tensor:
+def _launch_spmm(W: PaddedCSR, X: torch.Tensor, bias: torch.Tensor | None = None,
+                 halves: int | None = None) -> torch.Tensor:
+    """W·X (+ bias per row); halves: what _quad_halves said, if it was asked."""
     Y = torch.empty((W.nrows, X.shape[1]), dtype=torch.float32, device=X.device)
-    halves = _quad_halves(W, *X.shape)
+    if halves is None:
+        halves = _quad_halves(W, *X.shape)
     if halves:
         _lib.spmm_quad(W._view(), W._quads(halves), W.values, X, Y, bias)
         return Y
@@ -309,7 +333,8 @@ def _strip_sizes(W: PaddedCSR, N: int):
     if W.nnz * N < _STRIP_MIN_WORK or "seg" in _overrides or "dense_dw" in _overrides or \
             not _lib.FORCED_KNOBS.isdisjoint(("sddmm_g", "seg_lean", "seg_group")):
         return None
-    return W._strip_choice(N)
+    sizes = W._strip_choice(N)
+    return sizes if sizes and _recording_pays(W, N) else None
 
 
 def _launch_sddmm(W: PaddedCSR, dY: torch.Tensor, X: torch.Tensor, kernel: str,
@@ -411,7 +436,7 @@ def _spmm_backward(W: PaddedCSR, X: torch.Tensor, dY_f32: torch.Tensor, kernel: 
         else:
             if not fresh:
                 _lib.transpose_refresh(W.values, perm, WT.values)
-            dX = _launch_spmm(WT, dY_f32)
+            dX = _launch_spmm(WT, dY_f32, halves=0)
     return dW_values, dX
 
 
