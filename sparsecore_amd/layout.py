@@ -466,6 +466,18 @@ class PaddedCSR:
             v.own = own
         return v
 
+    def _skewed(self) -> bool:
+        """Whether more than one row in 32 is heavy (heavy_row_count; a random
+        mask's rows almost never are): for matrices below _ORDER_MIN_ROWS, whose
+        views do not count them. From the transpose's hint or one host read per
+        row_nnz; under capture, where none is possible, True."""
+        if self._heavy_hint is None:
+            if self._host_rows is None and torch.cuda.is_current_stream_capturing():
+                return True
+            nz = self._host_rows[1] if self._host_rows is not None else self._row_nnz.cpu().numpy()
+            self._heavy_hint = heavy_row_count(nz)
+        return 32 * self._heavy_hint > self._nrows
+
     def _dense_scratch(self, n_dense: int) -> torch.Tensor | None:
         """Scratch of the matrix-core path for n_dense dense rows; None for 0."""
         if not n_dense:
@@ -892,6 +904,9 @@ class PaddedCSR:
                                     self._row_nnz.to(device), self._row_cap.to(device),
                                     self._nnz, self._topology_version)
         out._host_rows = self._host_rows
+        if not self._on_device():  # counted where the rows are at hand
+            out._heavy_hint = heavy_row_count(self._row_nnz.numpy())
+            out._dense_hint = dense_row_count(self._row_nnz.numpy(), self._ncols)
         return out
 
     def cuda(self, device=None) -> "PaddedCSR":
@@ -1221,10 +1236,7 @@ def transposes_with_perm(ps, *, padding_ratio: float = 0.2):
         nnz_t = torch.empty(K, dtype=_I32, device=dev)
         cap_t = torch.empty(K, dtype=_I32, device=dev)
         _lib.transpose_count(view, padding_ratio, ws, rs_t, nnz_t, cap_t, caps[i:i + 1])
-        if K >= PaddedCSR._ORDER_MIN_ROWS:  # only scheduled views use the counts
-            _count_rows(nnz_t, p.nnz, p.nrows, caps[n + 2 * i:n + 2 * i + 2])
-        else:
-            caps[n + 2 * i:n + 2 * i + 2].zero_()
+        _count_rows(nnz_t, p.nnz, p.nrows, caps[n + 2 * i:n + 2 * i + 2])
         # the fill right behind the count, into arrays sized by a bound of
         # the capacity (as transpose_with_perm)
         bound = _capacity_bound(p.nnz, K, padding_ratio)

@@ -223,6 +223,34 @@ def _recording_pays(W: PaddedCSR, N: int) -> bool:
         W.nnz * N >= (_CAPTURED_MIN_WORK if N % 4 else _CAPTURED_MIN_WORK_ALIGNED)
 
 
+# The estimates behind quads and strips take rows of like length, and refuse
+# heavy rows, which only views from _ORDER_MIN_ROWS rows on count. Below that,
+# where more than one row in 32 is heavy (Zipf(0.5) and Zipf(1.1) row lengths,
+# 256 to 2000 rows, 784 to 4096 columns, 3% to 25%; each against slk_spmm or
+# slk_sddmm): at N a multiple of 4 quads are faster up to 512 rows (1.0-1.7x) and
+# at 3% (1.0-2.3x) but slower above (0.73-1.1x, most at 1024 x 2048, 10%: 271 ->
+# 370 us); at other N they are always faster (1.1-3.5x). Strips are slower at N a
+# multiple of 4 (0.45-1.06x: 2000 x 4096 at 3%, N = 2048: 94 -> 207 us), faster at
+# other N (1.06-4.7x), except below some 4e8 slots x N (2000 x 784 at 10%, N =
+# 1001: 52 -> 79).
+_SKEW_QUAD_MAX_ROWS = 512
+_SKEW_QUAD_MAX_DENSITY = 1 / 16
+_SKEW_STRIP_MIN_WORK = 400_000_000
+
+
+def _skewed(W: PaddedCSR) -> bool:
+    return W.nrows < W._ORDER_MIN_ROWS and W._skewed()
+
+
+def _skew_slows_quads(W: PaddedCSR, N: int) -> bool:
+    return N % 4 == 0 and W.nrows > _SKEW_QUAD_MAX_ROWS and \
+        W.nnz >= _SKEW_QUAD_MAX_DENSITY * W.nrows * W.ncols and _skewed(W)
+
+
+def _skew_slows_strips(W: PaddedCSR, N: int) -> bool:
+    return (N % 4 == 0 or W.nnz * N < _SKEW_STRIP_MIN_WORK) and _skewed(W)
+
+
 def _quad_halves(W: PaddedCSR, K: int, N: int) -> int:
     """64-column halves of the row quads (1 or 2) to run W on a K x N X with;
     0: slk_spmm."""
@@ -232,7 +260,7 @@ def _quad_halves(W: PaddedCSR, K: int, N: int) -> int:
     if W.nnz * N < _QUAD_MIN_WORK or "bin_shape" in _overrides or "spmm_phases" in _overrides:
         return 0
     halves = _lib.quad_halves(W._view(), N)
-    return halves if halves and _recording_pays(W, N) else 0
+    return halves if halves and _recording_pays(W, N) and not _skew_slows_quads(W, N) else 0
 
 
 def _spmm_view(W: PaddedCSR, X: torch.Tensor):
@@ -334,7 +362,7 @@ def _strip_sizes(W: PaddedCSR, N: int):
             not _lib.FORCED_KNOBS.isdisjoint(("sddmm_g", "seg_lean", "seg_group")):
         return None
     sizes = W._strip_choice(N)
-    return sizes if sizes and _recording_pays(W, N) else None
+    return sizes if sizes and _recording_pays(W, N) and not _skew_slows_strips(W, N) else None
 
 
 def _launch_sddmm(W: PaddedCSR, dY: torch.Tensor, X: torch.Tensor, kernel: str,
