@@ -493,19 +493,28 @@ double strip_cost(int64_t M, int64_t K, int64_t N, double density, const slk_str
            rounds * windows * (0.2 + stage + T.per_wave * (0.06 + step * steps));
 }
 
-// The same for slk_sddmm, from the shapes of strip_cost's measurement: what its
-// kernels reach there at best (slots x columns per ns), and the chain of windows
-// that one workgroup or wave runs however small the matrix. (Segment kernel: N
-// % 4 == 0 and N >= 1024, from 100000 slots; 4-slot segments below 1/16.)
+// The same for slk_sddmm: what its kernels reach (slots x columns per ns), and
+// the chain of windows that one workgroup or wave runs however small the matrix.
+// Segment kernel: N % 4 == 0 and N >= 1024, from 100000 slots; 4-slot segments
+// below 1/16. The rates are those of 423 shapes on which both sides were timed
+// (256 to 4096 rows, 384 to 4096 columns, 3% to 30%, N 256 to 8192): strips then
+// lose by 11% at most (768 x 4096 at 5%, N = 2048: 59 -> 66 us) and by over 3% on
+// seven. From 1.5 million slots below 1/8 the segment kernel gains (4096^2 at 10%,
+// N = 8192: 1254 us against 1402 in strips), as it does where rows hold over 40 of
+// 70000 to 100000 slots on the per-slot kernels (1000 x 768 at 10%, N = 1024: 19
+// against 23).
 double sddmm_estimate(const slk_csr* W, int64_t N, double density) {
     const double slots = W->total_capacity / 1.2, work = slots * N * 1e-3;
     double rate = 3.9, chain = 0.0;
     if (N % 4 == 0 && N >= 1024 && slots >= 1e5) {
-        rate = density < 0.0625 ? (4.0 * W->ncols * N >= (1 << 27) ? 5.6 : 4.5) : 7.6 + 13.5 * density;
+        if (density >= 0.0625) rate = 7.6 + 13.5 * density;
+        else if (4.0 * W->ncols * N >= (1 << 27)) rate = 5.6;
+        else rate = density >= 0.04 ? 5.2 : 4.5;
         if (slots >= 2e6) rate *= 1.3;
+        else if (slots >= 1.5e6 && density < 0.125) rate *= 1.2;
         chain = 1.25 * N / 64.0;
     } else if (N % 4 == 0) {
-        rate = N >= 1024 ? 4.3 : 3.75;
+        rate = N < 1024 ? 3.75 : slots >= 7e4 && slots >= 40.0 * W->nrows ? 5.0 : 4.3;
         chain = N / 150.0;
     }
     return 4.0 + std::fmax(work / rate * 1e-3, chain);

@@ -37,6 +37,21 @@ def test_strips_only_where_they_measured_faster(M, K, N, density, takes):
     assert (_lib.strip_choose(_view(M, K, density), N)[0] is not None) == takes
 
 
+@pytest.mark.parametrize("M,K,N,density,takes", [
+    # measured us, slk_sddmm against strips: where the segment kernel gains, and beside it
+    (4096, 4096, 8192, 0.1, False),   # 1254, 1402
+    (768, 4096, 1024, 0.05, False),   # 34, 40
+    (1000, 768, 1024, 0.1, False),    # 19, 23
+    (1537, 1000, 8192, 0.05, False),  # 128, 137
+    (4096, 384, 4096, 0.05, True),    # 130, 68
+    (256, 784, 8192, 0.25, True),     # 117, 94
+    (4096, 2048, 8192, 0.2, True),    # 1115, 983
+    (2000, 2048, 2048, 0.03, True),   # 63, 56
+])
+def test_strips_not_where_the_segment_kernel_gains(M, K, N, density, takes):
+    assert (_lib.strip_choose(_view(M, K, density), N)[0] is not None) == takes
+
+
 def test_strips_leave_skewed_and_dense_rows_alone():
     assert _lib.strip_choose(_view(2304, 768, 0.3), 8192)[0] is not None
     assert _lib.strip_choose(_view(2304, 768, 0.3, row_order=8, n_heavy_rows=1), 8192)[0] is None
