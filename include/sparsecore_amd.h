@@ -32,7 +32,7 @@
 extern "C" {
 #endif
 
-#define SLK_ABI_VERSION 17
+#define SLK_ABI_VERSION 18
 
 #if defined(__GNUC__)
 #define SLK_API __attribute__((visibility("default")))
@@ -296,6 +296,17 @@ SLK_API int slk_quad_build(const slk_csr* W, const int64_t* perm, int64_t halves
                    int64_t ws_words, int32_t* start, uint8_t* count, uint32_t* offset,
                    int32_t* slot, int64_t n_windows, int32_t* used, void* stream);
 
+/* The same in two steps, for large matrices: slk_quad_windows takes a quad's
+ * longest row for the sum of its four, up to four times what is used.
+ * slk_quad_count fills ws, start, count and used; used[nq], read on the host, is
+ * then the n_windows that offset and slot need for slk_quad_fill, which takes
+ * the same ws, start, count and used once (windows past n_windows are left out). */
+SLK_API int slk_quad_count(const slk_csr* W, int64_t halves, int32_t* ws, int64_t ws_words,
+                   int32_t* start, uint8_t* count, int32_t* used, void* stream);
+SLK_API int slk_quad_fill(const slk_csr* W, const int64_t* perm, int64_t halves, int32_t* ws,
+                  int64_t ws_words, int32_t* start, uint8_t* count, uint32_t* offset,
+                  int32_t* slot, int64_t n_windows, int32_t* used, void* stream);
+
 /* slk_spmm (slk_spmm_bias with a bias; NULL: none) through W's quads, the same
  * bits, for N in [4, 2^22]. values is what the quads' slots index (W's own, or
  * with perm those of the matrix that W is the transpose of; W->values is not
@@ -352,7 +363,7 @@ SLK_API int slk_strip_words(const slk_csr* W, const slk_strips* T, int64_t* word
 /* Builds them on the device: three launches, no host read. used: 1 word.     */
 SLK_API int slk_strip_build(const slk_csr* W, const slk_strips* T, int32_t* items, int32_t* rel,
                     int32_t* used, int32_t* ws, void* stream);
-/* Bytes of slk_sddmm_strips' workspace: a copy of X, padded to 64 columns.   */
+/* Bytes of slk_sddmm_strips' workspace: a copy of X, padded to 128 columns.  */
 SLK_API int64_t slk_strip_layout_bytes(int64_t ncols, int64_t N);
 /* slk_sddmm (SLK_DW_SIMD; with dbias slk_sddmm_bias) for W's strips, the same
  * bits; slots of rows before `first` are left alone. N in [1, 2^21]. ws is

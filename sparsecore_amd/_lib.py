@@ -21,7 +21,7 @@ from pathlib import Path
 import torch
 
 LIB_PATH = Path(__file__).resolve().parent / "_lib" / "libsparsecore_amd.so"
-ABI_VERSION = 17
+ABI_VERSION = 18
 
 SLK_OK, SLK_EINVAL, SLK_EDEVICE = 0, 1, 2
 SLK_DW_SIMD, SLK_DW_SCALAR = 0, 1
@@ -72,6 +72,8 @@ EXPORTS = (
     "slk_quad_windows",
     "slk_quad_chunks",
     "slk_quad_halves",
+    "slk_quad_count",
+    "slk_quad_fill",
     "slk_quad_build",
     "slk_spmm_quad",
     "slk_strip_choose",
@@ -217,7 +219,9 @@ def _declare(lib) -> None:
     lib.slk_quad_windows.argtypes = [_csrp, _i64]
     lib.slk_quad_chunks.argtypes = [_i64, _i64]
     lib.slk_quad_halves.argtypes = [_csrp, _i64]
-    lib.slk_quad_build.argtypes = [_csrp, _vp, _i64, _vp, _i64, _vp, _vp, _vp, _vp, _i64, _vp, _vp]
+    lib.slk_quad_count.argtypes = [_csrp, _i64, _vp, _i64, _vp, _vp, _vp, _vp]
+    for fn in (lib.slk_quad_fill, lib.slk_quad_build):
+        fn.argtypes = [_csrp, _vp, _i64, _vp, _i64, _vp, _vp, _vp, _vp, _i64, _vp, _vp]
     lib.slk_spmm_quad.argtypes = [_csrp, ctypes.POINTER(QuadView), _vp, _vp, _vp, _i64, _i64, _vp,
                                   _vp, _vp]
     stripp = ctypes.POINTER(StripView)
@@ -460,6 +464,17 @@ def backward_fused(view: CsrView, viewT: CsrView, perm: torch.Tensor, dY: torch.
         _raise(rc)
 
 
+# Quads whose bound (quad_bytes) is larger are sized by the exact count of their
+# windows, read on the host between the count and the fill (16384^2 at 5%: 654 MB
+# bound; the read waits for the queue, some 20 us of a pass of milliseconds).
+QUAD_READ_BYTES = 128 << 20
+
+
+def quad_bytes(view: CsrView, halves: int) -> int:
+    """A bound of the bytes that view's quads keep: offset and slot of their windows."""
+    return 512 * int(load().slk_quad_windows(ctypes.byref(view), halves))
+
+
 def quad_build(view: CsrView, perm: torch.Tensor | None, halves: int, device) -> QuadView:
     """view's row quads (slk_quad_build) as a QuadView that holds its arrays; with
     perm, for the values of the matrix that view's is the transpose of."""
@@ -472,9 +487,16 @@ def quad_build(view: CsrView, perm: torch.Tensor | None, halves: int, device) ->
     ws = torch.empty(words, **i32)
     start, used = torch.empty(nc * nq, **i32), torch.empty(nq + 1, **i32)
     count = torch.empty(nc * nq, dtype=torch.uint8, device=device)
+    stream, fill = stream_of(start), lib.slk_quad_build
+    if quad_bytes(view, halves) > QUAD_READ_BYTES and not torch.cuda.is_current_stream_capturing():
+        rc = lib.slk_quad_count(ctypes.byref(view), halves, ptr(ws), words, ptr(start), ptr(count),
+                                ptr(used), stream)
+        if rc:
+            _raise(rc)
+        n, fill = int(used[nq]), lib.slk_quad_fill
     offset, slot = torch.empty(64 * n, **i32), torch.empty(64 * n, **i32)
-    rc = lib.slk_quad_build(ctypes.byref(view), ptr(perm), halves, ptr(ws), words, ptr(start),
-                            ptr(count), ptr(offset), ptr(slot), n, ptr(used), stream_of(start))
+    rc = fill(ctypes.byref(view), ptr(perm), halves, ptr(ws), words, ptr(start), ptr(count),
+              ptr(offset), ptr(slot), n, ptr(used), stream)
     if rc:
         _raise(rc)
     arrays = (start, count, offset, slot, used)

@@ -393,7 +393,7 @@ __global__ __launch_bounds__(256) void quad_fill_kernel(
     const int32_t* __restrict__ col, const int64_t* __restrict__ perm,
     const int32_t* __restrict__ rel, const int32_t* __restrict__ total,
     int32_t* __restrict__ qstart, const uint8_t* __restrict__ qcount, uint32_t* __restrict__ qoff,
-    int32_t* __restrict__ qslot, int32_t row_bytes) {
+    int32_t* __restrict__ qslot, int64_t n_windows, int32_t row_bytes) {
     const int64_t q = blockIdx.x;
     const int lane = threadIdx.x & (kWave - 1), r = lane >> 4, l16 = lane & 15;
     const int64_t row = 4 * q + r;
@@ -405,7 +405,7 @@ __global__ __launch_bounds__(256) void quad_fill_kernel(
         const int32_t first = qstart[at] + base, n = qcount[at];
         const int32_t nw = n > 16 ? (n + 15) >> 4 : 1;
         const int32_t lo = mine[ch], hi = mine[ch + 1];
-        for (int32_t iw = 0; iw < nw; ++iw) {
+        for (int32_t iw = 0; iw < nw && first + iw < n_windows; ++iw) {
             const int32_t s = lo + 16 * iw + l16;
             const int64_t i = static_cast<int64_t>(first + iw) * kWave + lane;
             uint32_t off = kZeroOff;
@@ -535,48 +535,83 @@ extern "C" int64_t slk_quad_halves(const slk_csr* W, int64_t N) {
     return best != 0 && least < 0.9 * spmm_estimate(W, N) ? best : 0;
 }
 
+namespace slk {
+namespace {
+
+// What every part of the build checks; the quads and chunks.
+int quad_extent(const slk_csr* W, int64_t halves, int64_t ws_words, const char* who, int64_t* nq,
+                int64_t* nch) {
+    clear_error();
+    if (int rc = validate_csr(W, who)) return rc;
+    const std::string at = std::string(who) + ": ";
+    if (!halves_ok(halves)) return fail(SLK_EINVAL, at + "halves must be 1 or 2");
+    if (W->nrows == 0 || W->ncols == 0) return fail(SLK_EINVAL, at + "empty matrix");
+    *nq = ceil_div(W->nrows, int64_t{4});
+    *nch = slk_quad_chunks(W->ncols, halves);
+    if (*nch > kMaxChunks) return fail(SLK_EINVAL, at + "too many columns");
+    if (*nq > INT32_MAX) return fail(SLK_EINVAL, at + "too many rows");
+    const int64_t need = *nq * 4 * (*nch + 1);
+    if (ws_words < need)
+        return fail(SLK_EINVAL, at + "workspace of " + std::to_string(ws_words) + " words, needs " +
+                                    std::to_string(need));
+    return SLK_OK;
+}
+
+}  // namespace
+}  // namespace slk
+
+extern "C" int slk_quad_count(const slk_csr* W, int64_t halves, int32_t* ws, int64_t ws_words,
+                              int32_t* start, uint8_t* count, int32_t* used, void* stream) {
+    using namespace slk;
+    int64_t nq = 0, nch = 0;
+    if (int rc = quad_extent(W, halves, ws_words, "quad_build", &nq, &nch)) return rc;
+    if (ws == nullptr || start == nullptr || count == nullptr || used == nullptr)
+        return fail(SLK_EINVAL, "quad_build: NULL output");
+    hipStream_t st = as_stream(stream);
+    auto* kernel = halves == 2 ? quad_count_kernel<chunk_rows(2)> : quad_count_kernel<chunk_rows(1)>;
+    hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(nq)), dim3(256),
+                       static_cast<unsigned>(16 * (nch + 1)), st, W->nrows, nq,
+                       static_cast<int32_t>(nch), W->row_start, W->row_nnz, W->col_indices, ws,
+                       start, count, used);
+    if (int rc = check_launch("quad_build: count")) return rc;
+    hipLaunchKernelGGL(quad_scan_kernel, dim3(1), dim3(1024), 0, st, nq, used);
+    return check_launch("quad_build: scan");
+}
+
+extern "C" int slk_quad_fill(const slk_csr* W, const int64_t* perm, int64_t halves, int32_t* ws,
+                             int64_t ws_words, int32_t* start, uint8_t* count, uint32_t* offset,
+                             int32_t* slot, int64_t n_windows, int32_t* used, void* stream) {
+    using namespace slk;
+    int64_t nq = 0, nch = 0;
+    if (int rc = quad_extent(W, halves, ws_words, "quad_build", &nq, &nch)) return rc;
+    if (n_windows < 1 || n_windows > INT32_MAX)
+        return fail(SLK_EINVAL, "quad_build: no or too many windows");
+    if (ws == nullptr || start == nullptr || count == nullptr || offset == nullptr ||
+        slot == nullptr || used == nullptr)
+        return fail(SLK_EINVAL, "quad_build: NULL output");
+    auto* kernel = halves == 2 ? quad_fill_kernel<chunk_rows(2)> : quad_fill_kernel<chunk_rows(1)>;
+    hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(nq)), dim3(256), 0, as_stream(stream),
+                       W->nrows, nq, static_cast<int32_t>(nch), W->row_start, W->col_indices, perm,
+                       ws, used, start, count, offset, slot, n_windows,
+                       static_cast<int32_t>(256 * halves));
+    return check_launch("quad_build: fill");
+}
+
 extern "C" int slk_quad_build(const slk_csr* W, const int64_t* perm, int64_t halves, int32_t* ws,
                               int64_t ws_words, int32_t* start, uint8_t* count, uint32_t* offset,
                               int32_t* slot, int64_t n_windows, int32_t* used, void* stream) {
     using namespace slk;
-    clear_error();
-    if (int rc = validate_csr(W, "quad_build")) return rc;
-    if (!halves_ok(halves)) return fail(SLK_EINVAL, "quad_build: halves must be 1 or 2");
-    const int64_t M = W->nrows, K = W->ncols;
-    if (M == 0 || K == 0) return fail(SLK_EINVAL, "quad_build: empty matrix");
-    const int64_t nq = ceil_div(M, int64_t{4}), nch = slk_quad_chunks(K, halves);
-    if (nch > kMaxChunks) return fail(SLK_EINVAL, "quad_build: too many columns");
-    const int64_t need = nq * 4 * (nch + 1);
-    if (ws_words < need || n_windows < slk_quad_windows(W, halves))
-        return fail(SLK_EINVAL, "quad_build: workspace of " + std::to_string(ws_words) +
-                                    " words and " + std::to_string(n_windows) +
-                                    " windows, needs " + std::to_string(need) + " and " +
+    int64_t nq = 0, nch = 0;
+    if (int rc = quad_extent(W, halves, ws_words, "quad_build", &nq, &nch)) return rc;
+    if (n_windows < slk_quad_windows(W, halves))
+        return fail(SLK_EINVAL, "quad_build: workspace of " + std::to_string(n_windows) +
+                                    " windows, needs " +
                                     std::to_string(slk_quad_windows(W, halves)));
     if (n_windows > INT32_MAX) return fail(SLK_EINVAL, "quad_build: too many windows");
-    if (nq > INT32_MAX) return fail(SLK_EINVAL, "quad_build: too many rows");
-    if (ws == nullptr || start == nullptr || count == nullptr || offset == nullptr ||
-        slot == nullptr || used == nullptr)
-        return fail(SLK_EINVAL, "quad_build: NULL output");
-    hipStream_t st = as_stream(stream);
-    const dim3 grid(static_cast<unsigned>(nq));
-    const unsigned lds = static_cast<unsigned>(16 * (nch + 1));
-#define SLK_QUAD_BUILD(H)                                                                         \
-    do {                                                                                          \
-        constexpr int KC = chunk_rows(H);                                                         \
-        hipLaunchKernelGGL(quad_count_kernel<KC>, grid, dim3(256), lds, st, M, nq,                \
-                           static_cast<int32_t>(nch), W->row_start, W->row_nnz, W->col_indices,   \
-                           ws, start, count, used);                                               \
-        if (int rc = check_launch("quad_build: count")) return rc;                                \
-        hipLaunchKernelGGL(quad_scan_kernel, dim3(1), dim3(1024), 0, st, nq, used);               \
-        if (int rc = check_launch("quad_build: scan")) return rc;                                 \
-        hipLaunchKernelGGL(quad_fill_kernel<KC>, grid, dim3(256), 0, st, M, nq,                   \
-                           static_cast<int32_t>(nch), W->row_start, W->col_indices, perm, ws,     \
-                           used, start, count, offset, slot, 256 * H);                            \
-    } while (0)
-    if (halves == 2) SLK_QUAD_BUILD(2);
-    else SLK_QUAD_BUILD(1);
-#undef SLK_QUAD_BUILD
-    return check_launch("quad_build: fill");
+    if (offset == nullptr || slot == nullptr) return fail(SLK_EINVAL, "quad_build: NULL output");
+    if (int rc = slk_quad_count(W, halves, ws, ws_words, start, count, used, stream)) return rc;
+    return slk_quad_fill(W, perm, halves, ws, ws_words, start, count, offset, slot, n_windows, used,
+                         stream);
 }
 
 extern "C" int slk_spmm_quad(const slk_csr* W, const slk_quads* Q, const float* values,

@@ -260,7 +260,26 @@ def _quad_halves(W: PaddedCSR, K: int, N: int) -> int:
     if W.nnz * N < _QUAD_MIN_WORK or "bin_shape" in _overrides or "spmm_phases" in _overrides:
         return 0
     halves = _lib.quad_halves(W._view(), N)
-    return halves if halves and _recording_pays(W, N) and not _skew_slows_quads(W, N) else 0
+    if not halves or not _recording_pays(W, N) or _skew_slows_quads(W, N):
+        return 0
+    if torch.cuda.is_current_stream_capturing() and \
+            _lib.quad_bytes(W._view(), halves) > _lib.QUAD_READ_BYTES:
+        return 0  # a graph cannot read their exact size, and would hold the bound
+    return halves
+
+
+def _spmm_quads(W: PaddedCSR, values: torch.Tensor, X: torch.Tensor, Y: torch.Tensor,
+                halves: int, perm: torch.Tensor | None = None,
+                bias: torch.Tensor | None = None) -> bool:
+    """Y = W·X (+ bias) through W's row quads. False, with nothing launched and
+    W's quads given up, where the memory for them is not to be had: slk_spmm needs
+    none."""
+    try:
+        _lib.spmm_quad(W._view(), W._quads(halves, perm), values, X, Y, bias)
+    except torch.OutOfMemoryError:
+        W._quads_kept = (-1, {})
+        return False
+    return True
 
 
 def _spmm_view(W: PaddedCSR, X: torch.Tensor):
@@ -287,8 +306,7 @@ def _launch_spmm(W: PaddedCSR, X: torch.Tensor, bias: torch.Tensor | None = None
     Y = torch.empty((W.nrows, X.shape[1]), dtype=torch.float32, device=X.device)
     if halves is None:
         halves = _quad_halves(W, *X.shape)
-    if halves:
-        _lib.spmm_quad(W._view(), W._quads(halves), W.values, X, Y, bias)
+    if halves and _spmm_quads(W, W.values, X, Y, halves, bias=bias):
         return Y
     _lib.spmm(_spmm_view(W, X), X, Y, bias)
     return Y
@@ -371,8 +389,11 @@ def _launch_sddmm(W: PaddedCSR, dY: torch.Tensor, X: torch.Tensor, kernel: str,
     order = _lib.SLK_DW_SCALAR if kernel == "scalar" else _lib.SLK_DW_SIMD
     sizes = _strip_sizes(W, X.shape[1]) if order == _lib.SLK_DW_SIMD else None
     if sizes:
-        _lib.sddmm_strips(W._view(), W._strips(sizes), dY, X, dW, dbias)
-        return dW
+        try:
+            _lib.sddmm_strips(W._view(), W._strips(sizes), dY, X, dW, dbias)
+            return dW
+        except torch.OutOfMemoryError:  # for the strips or their copy of X
+            W._strips_kept = (-1, {})
     view = _sddmm_view(W, X) if order == _lib.SLK_DW_SIMD else W._view()
     _lib.sddmm(view, dY, X, dW, order, dbias)
     return dW
@@ -460,8 +481,8 @@ def _spmm_backward(W: PaddedCSR, X: torch.Tensor, dY_f32: torch.Tensor, kernel: 
         halves = _quad_halves(WT, *dY_f32.shape)
         if halves:  # through W's values: no refresh of WT's
             dX = torch.empty((W.ncols, dY_f32.shape[1]), dtype=torch.float32, device=W.device)
-            _lib.spmm_quad(WT._view(), WT._quads(halves, perm), W.values, dY_f32, dX)
-        else:
+        if not halves or not _spmm_quads(WT, W.values, dY_f32, dX, halves, perm):
+            dX = None
             if not fresh:
                 _lib.transpose_refresh(W.values, perm, WT.values)
             dX = _launch_spmm(WT, dY_f32, halves=0)

@@ -170,3 +170,27 @@ def test_quads_built_under_capture_stay_with_the_graph(dev, quad):
         torch.cuda.synchronize()
         quad(1)
         assert_bits_equal(Y.cpu().numpy(), ops._launch_spmm(W, X).cpu().numpy(), f"replay {step}")
+
+
+@pytest.mark.parametrize("halves", [1, 2])
+@pytest.mark.parametrize("M,K", [(1, 1), (66, 253), (130, 700)])
+def test_quads_sized_by_their_count_match_the_bound_sized(dev, monkeypatch, quad, halves, M, K):
+    """Above QUAD_READ_BYTES (here: always) offset and slot hold the windows used
+    and no more; the arrays, of a matrix and of its transpose, and the product
+    are the same."""
+    print(f"[quad exact size] {M}x{K} halves={halves}", flush=True)
+    c = _mixed(M, K, seed=M + K)
+    X = _t(np.random.default_rng(M).standard_normal((K, 68)).astype(np.float32), dev)
+    W = from_oracle(c, dev)
+    WT, perm, _ = ops._transpose_entry(W)
+    bound = [W._quads(halves), WT._quads(halves, perm)]
+    monkeypatch.setattr(_lib, "QUAD_READ_BYTES", 0)
+    W._quads_kept = WT._quads_kept = (-1, {})
+    for b, q in zip(bound, (W._quads(halves), WT._quads(halves, perm))):
+        n = int(b.arrays[4][-1])
+        assert q.n_windows == n <= b.n_windows
+        for i, name in enumerate(("start", "count", "offset", "slot", "used")):
+            want = b.arrays[i] if i not in (2, 3) else b.arrays[i][:64 * n]
+            assert_bits_equal(q.arrays[i].cpu().numpy(), want.cpu().numpy(), name)
+    quad(halves)
+    assert_bits_equal(ops._launch_spmm(W, X).cpu().numpy(), oracle.spmm(c, X.cpu().numpy()), "Y")
