@@ -260,44 +260,20 @@ __global__ __launch_bounds__(kSpmmBlock) void spmm_wave_kernel(
     }
 }
 
-// Few columns of X: waves are few (3072 rows at N = 8: 1.5 per CU) and a row's
-// time is its chain of dependent loads, metadata then X, so the chain is cut:
-// the L lanes of a row load a batch of kBatch slots' metadata together, one
-// batch ahead, broadcast it by shuffles, and have the whole batch's gathers in
-// flight at once. The last batch is padded with the row's last slot, whose
-// extra products are dropped. 3072 x 768 at 10%, N = 8: 14.4 -> 8.6 us, 768 x 3072 44 -> 23 against
-// eight slots at a time with the remainder one by one, each lane loading all
-// metadata itself.
-template <int L, int VEC>
-__global__ __launch_bounds__(kSpmmBlock) void spmm_group_kernel(
-    int64_t M, int64_t N, int64_t nitems, const int32_t* __restrict__ order,
-    const int32_t* __restrict__ row_start, const int32_t* __restrict__ row_nnz,
-    const int32_t* __restrict__ col, const float* __restrict__ val,
-    const float* __restrict__ X, const float* __restrict__ bias, float* __restrict__ Y) {
-    typedef VecIO<VEC> IO;
-    constexpr int kBatch = 16;
-    constexpr int J = L < kBatch ? kBatch / L : 1;  // slots a lane loads of a batch
-    static_assert(L >= 8, "the lanes of a row share its metadata");
-    constexpr int kItemsPerWave = kWave / L;
-    const int lane = threadIdx.x & (kWave - 1), l = lane % L;
-    const int64_t item = wave_id() * kItemsPerWave + lane / L;
-    const bool valid = item < nitems;
-    const int64_t tile = valid ? item / M : 0;
-    const int64_t r = valid ? item - tile * M : 0;
-    const int64_t row = order != nullptr ? order[r] : r;
-    const int64_t n0 = (tile * L + l) * VEC;
-    const bool active = valid && n0 < N;
-
-    const int32_t nnz = valid ? row_nnz[row] : 0;
-    const int32_t* c_ptr = col + row_start[row];
-    const float* v_ptr = val + row_start[row];
-    // lanes without an item or past N read the first columns and store nothing
-    const float* xb = X + (active ? n0 : 0);
-
-    float acc[VEC];
-#pragma unroll
-    for (int e = 0; e < VEC; ++e) acc[e] = 0.0f;
-
+// Few columns of X (N <= 32): a row takes L lanes, lane l its column l. A row's
+// time is its chain of dependent loads, metadata then X, so the chain is cut: its
+// L lanes load a batch of B slots' metadata together, one batch ahead, broadcast
+// it by shuffles, and have the whole batch's gathers in flight at once. The last
+// batch is padded with the row's last slot, whose extra products are dropped.
+// PART: lanes past N gather nothing (65536 rows of 20 slots, N = 5: 13.3 us with
+// repeats of column 0, 9.1 without; N = 8, no such lane: 9.0, 9.2 with the test).
+template <int L, int B, bool PART>
+__device__ __forceinline__ float group_row(int32_t nnz, const int32_t* __restrict__ c_ptr,
+                                           const float* __restrict__ v_ptr,
+                                           const float* __restrict__ xb, int64_t N, int l,
+                                           bool active) {
+    constexpr int J = L < B ? B / L : 1;  // slots a lane loads of a batch
+    float acc = 0.0f;
     int32_t c[J], cn[J];
     float v[J], vn[J];
 #pragma unroll
@@ -315,22 +291,23 @@ __global__ __launch_bounds__(kSpmmBlock) void spmm_group_kernel(
         }
     };
     fetch(0, c, v);
-    for (int32_t s = 0; __any(s < nnz); s += kBatch) {  // every lane: the shuffles need them
-        fetch(s + kBatch, cn, vn);
-        typename IO::T x[kBatch];  // (some row has slots here, so X has a row 0)
+    bool more = __any(0 < nnz);
+    for (int32_t s = 0; more; s += B) {  // every lane: the shuffles need them
+        more = __any(s + B < nnz);
+        if (more) fetch(s + B, cn, vn);
+        int32_t cu[B];
+        float x[B];  // (some row has slots here, so X has a row 0)
 #pragma unroll
-        for (int u = 0; u < kBatch; ++u) {
-            const int32_t cu = __shfl(c[u / L], u % L, L);
-            x[u] = IO::load(xb + static_cast<int64_t>(cu) * N);
+        for (int u = 0; u < B; ++u) cu[u] = L == 1 ? c[u % J] : __shfl(c[u / L], u % L, L);
+        if (!PART || active) {
+#pragma unroll
+            for (int u = 0; u < B; ++u) x[u] = xb[static_cast<int64_t>(cu[u]) * N];
         }
 #pragma unroll
-        for (int u = 0; u < kBatch; ++u) {
-            const float vu = __shfl(v[u / L], u % L, L);
-#pragma unroll
-            for (int e = 0; e < VEC; ++e) {
-                const float f = __builtin_fmaf(vu, IO::get(x[u], e), acc[e]);
-                acc[e] = s + u < nnz ? f : acc[e];
-            }
+        for (int u = 0; u < B; ++u) {
+            const float vu = L == 1 ? v[u % J] : __shfl(v[u / L], u % L, L);
+            const float f = __builtin_fmaf(vu, x[u], acc);
+            acc = s + u < nnz ? f : acc;
         }
 #pragma unroll
         for (int j = 0; j < J; ++j) {
@@ -338,10 +315,33 @@ __global__ __launch_bounds__(kSpmmBlock) void spmm_group_kernel(
             v[j] = vn[j];
         }
     }
-    if (active) {
-        if (bias != nullptr) add_bias<VEC>(acc, bias[row]);
-        IO::store(Y + row * N + n0, acc);
-    }
+    return acc;
+}
+
+// The batch follows the wave's longest row, so that rows of a few slots pay for
+// few gathers; with one or two lanes a row it stops at 8 (registers).
+template <int L, bool PART>
+__global__ __launch_bounds__(kSpmmBlock) void spmm_group_kernel(
+    int64_t M, int64_t N, const int32_t* __restrict__ order,
+    const int32_t* __restrict__ row_start, const int32_t* __restrict__ row_nnz,
+    const int32_t* __restrict__ col, const float* __restrict__ val,
+    const float* __restrict__ X, const float* __restrict__ bias, float* __restrict__ Y) {
+    const int lane = threadIdx.x & (kWave - 1), l = lane % L;
+    const int64_t r = wave_id() * (kWave / L) + lane / L;
+    const bool valid = r < M;
+    const int64_t row = !valid ? 0 : order != nullptr ? order[r] : r;
+    const bool active = valid && l < N;
+    const int32_t nnz = valid ? row_nnz[row] : 0;
+    const int32_t* c = col + row_start[row];
+    const float* v = val + row_start[row];
+    // lanes without a row or past N read column 0 and store nothing
+    const float* x = X + (active ? l : 0);
+    float acc;
+    if (L >= 4 && __any(nnz > 8)) acc = group_row<L, 16, PART>(nnz, c, v, x, N, l, active);
+    else if (__any(nnz > 4)) acc = group_row<L, 8, PART>(nnz, c, v, x, N, l, active);
+    else if (__any(nnz > 2)) acc = group_row<L, 4, PART>(nnz, c, v, x, N, l, active);
+    else acc = group_row<L, 2, PART>(nnz, c, v, x, N, l, active);
+    if (active) Y[row * N + l] = bias != nullptr ? acc + bias[row] : acc;
 }
 
 // ───────────────────────── LDS-staged kernel ────────────────────────────────
@@ -971,25 +971,45 @@ int launch_wave(const slk_csr* W, const float* X, int64_t N, const float* bias, 
     return check_launch("spmm");
 }
 
-template <int L, int VEC>
-int launch_group(const slk_csr* W, const float* X, int64_t N, const float* bias, float* Y,
-                 hipStream_t st) {
-    const int64_t M = W->nrows;
-    const int64_t nitems = M * ceil_div(N, static_cast<int64_t>(L) * VEC);
+template <int L>
+int launch_group(const slk_csr* W, const int32_t* order, const float* X, int64_t N,
+                 const float* bias, float* Y, hipStream_t st) {
     int64_t blocks;
-    if (int rc = launch_blocks(ceil_div(nitems, kWave / L), &blocks)) return rc;
-    hipLaunchKernelGGL((spmm_group_kernel<L, VEC>), dim3(static_cast<unsigned>(blocks)),
-                       dim3(kSpmmBlock), 0, st, M, N, nitems, W->row_order, W->row_start,
-                       W->row_nnz, W->col_indices, W->values, X, bias, Y);
+    if (int rc = launch_blocks(ceil_div(W->nrows, int64_t{kWave / L}), &blocks)) return rc;
+    auto* kernel = spmm_group_kernel<L, false>;
+    if constexpr (L >= 8)
+        if (N < L) kernel = spmm_group_kernel<L, true>;
+    hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(blocks)), dim3(kSpmmBlock), 0, st, W->nrows,
+                       N, order, W->row_start, W->row_nnz, W->col_indices, W->values, X, bias, Y);
     return check_launch("spmm");
 }
 
-int launch_group_L(int L, const slk_csr* W, const float* X, int64_t N, const float* bias,
-                   float* Y, hipStream_t st) {
+// N <= 32. Natural order reads the metadata of short rows in sequence; longest
+// rows first, at 8 lanes or more each, where more than one row in 32 is heavy and
+// rows hold over 5.5 slots on average (of a random mask's rows at 2 slots 14% are
+// heavy, at 4 5%, at 6 up to 2%; of Zipf(1.1) rows 6% and up), or where `order`
+// says which rows the view has (all_rows false). Lanes: the least power of two
+// that holds N, but 4 unless the matrix is large and its rows hold 4 slots or
+// fewer. At N = 1, by lanes per row, batch and order (8 lanes, batches of 16,
+// longest first; a lane per row, eight slots and then one at a time; this):
+// 2^20 rows of 1 slot 60, 5.5, 6.4 us; of 1 on average 65, 59, 11.5; 2304 rows
+// of 150 12, 22, 11.
+int spmm_group(const slk_csr* W, bool all_rows, const float* X, int64_t N, const float* bias,
+               float* Y, hipStream_t st) {
+    const int64_t M = W->nrows;
+    // (a row's capacity is 1.2 times its slots)
+    const bool longer = W->total_capacity > 4.8 * M;
+    const bool skewed = W->total_capacity > 6.6 * M && 32 * W->n_heavy_rows > M;
+    const int32_t* order = skewed || !all_rows ? W->row_order : nullptr;
+    int L = skewed ? 8 : M <= 16384 || longer ? 4 : 1;
+    while (L < N) L <<= 1;
     switch (L) {
-        case 8: return launch_group<8, 1>(W, X, N, bias, Y, st);
-        case 16: return launch_group<16, 1>(W, X, N, bias, Y, st);
-        default: return launch_group<32, 1>(W, X, N, bias, Y, st);
+        case 1: return launch_group<1>(W, order, X, N, bias, Y, st);
+        case 2: return launch_group<2>(W, order, X, N, bias, Y, st);
+        case 4: return launch_group<4>(W, order, X, N, bias, Y, st);
+        case 8: return launch_group<8>(W, order, X, N, bias, Y, st);
+        case 16: return launch_group<16>(W, order, X, N, bias, Y, st);
+        default: return launch_group<32>(W, order, X, N, bias, Y, st);
     }
 }
 
@@ -1217,8 +1237,10 @@ int spmm_split_two_queues(const slk_csr* W, int64_t T, const float* X, int64_t N
     return rc;
 }
 
+// all_rows: W's rows are the matrix's (row_order then only orders them), not a
+// part of them that row_order lists.
 int spmm_impl(const slk_csr* W, const float* X, int64_t K, int64_t N, const float* bias,
-              float* Y, void* stream, bool transposed_out = false) {
+              float* Y, void* stream, bool transposed_out = false, bool all_rows = true) {
     clear_error();
     if (int rc = validate_csr(W, "spmm")) return rc;
     if (N < 0 || K < 0) return fail(SLK_EINVAL, "spmm: negative X shape");
@@ -1266,7 +1288,7 @@ int spmm_impl(const slk_csr* W, const float* X, int64_t K, int64_t N, const floa
             if (done || rc != SLK_OK) return rc;
         }
         if (int rc = spmm_dense_rows(W, X, K, N, bias, Y, st)) return rc;
-        return spmm_impl(&rest, X, K, N, bias, Y, stream);
+        return spmm_impl(&rest, X, K, N, bias, Y, stream, false, false);
     }
     const uintptr_t align = reinterpret_cast<uintptr_t>(X) | reinterpret_cast<uintptr_t>(Y);
     const int64_t M = W->nrows;
@@ -1349,15 +1371,8 @@ int spmm_impl(const slk_csr* W, const float* X, int64_t K, int64_t N, const floa
         (vec != 1 && vec != 2 && vec != 4)) {
         vec = 1;
     }
-    if (N < kWave * vec) {
-        // Narrow X: pack several rows per wave, at least 8 lanes each (at N = 1
-        // seven only share the loads of the metadata: 2304 x 768 at 30% 37 ->
-        // 18 us against a lane per row).
-        int L = 8;
-        while (L < 32 && L < N) L <<= 1;
-        if (L < kWave && L >= N) return launch_group_L(L, W, X, N, bias, Y, st);
-        vec = 1;
-    }
+    if (N <= kWave / 2) return spmm_group(W, all_rows, X, N, bias, Y, st);
+    if (N < kWave * vec) vec = 1;
     if (vec == 4 && W->phase_lo != nullptr && W->n_phases > 1) return launch_phased4(W, X, N, bias, Y, st);
     if (vec == 4) return launch_wave<4>(W, X, N, bias, Y, st);
     if (vec == 2) return launch_wave<2>(W, X, N, bias, Y, st);
