@@ -25,8 +25,8 @@
 //    next chunk's first one at a chunk's end — is in flight while the current
 //    one is consumed), so a wave keeps 2U gathers outstanding instead of
 //    waiting once per slot, and never drains at a chunk boundary.
-//  * spmm_group_kernel — several items per wave (L < 64 lanes each) for
-//    narrow X (N < 64): the lanes of a row share its metadata.
+//  * spmm_group_kernel — several rows per wave (L <= 32 lanes each) for
+//    narrow X (N <= 32): the lanes of a row share its metadata.
 //
 // VEC (floats per lane) is chosen so that small problems still launch
 // enough waves to hide gather latency; large problems use 16-byte gathers.

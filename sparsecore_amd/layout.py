@@ -185,28 +185,41 @@ def _check_host(nrows, ncols, values, col, rs, nnz, cap) -> str:
 #  PaddedCSR
 # ─────────────────────────────────────────────────────────────────────
 
+def _raw_stream(index: int) -> int:
+    return torch._C._cuda_getCurrentRawStream(index)
+
+
 class _Built:
     """Device arrays that a lazy build has queued on the current stream, kept
-    for later calls on any stream: `event` is recorded behind the build."""
+    for later calls on any stream."""
 
-    __slots__ = ("value", "arrays", "stream", "event")
+    __slots__ = ("value", "arrays", "device", "stream", "joined")
 
     def __init__(self, value, arrays):
-        stream = torch.cuda.current_stream(arrays[0].device)
-        self.value, self.arrays, self.stream = value, arrays, stream.cuda_stream
-        # (what a capture builds is not kept, so nothing waits for it)
-        self.event = None if torch.cuda.is_current_stream_capturing() else stream.record_event()
+        self.value, self.arrays, self.device = value, arrays, arrays[0].device
+        self.stream = _raw_stream(self.device.index)
+        self.joined = {self.stream}
+
+    def elsewhere(self) -> bool:
+        """Whether the current stream is another one than the build's."""
+        return _raw_stream(self.device.index) != self.stream
 
     def join(self) -> None:
-        """Orders the current stream behind the build. The allocator is told of
-        a stream other than the build's, so that arrays dropped by their matrix
-        are not given away while that stream still reads them."""
-        if _lib.stream_of(self.arrays[0]) == self.stream:
+        """Orders the current stream behind the build, the first time that it is
+        another one than the build's, and names it to the allocator, so that
+        arrays dropped by their matrix are not given away while it still reads
+        them. The event is recorded now and not at the build, which most
+        matrices' calls never leave the stream of (an event in the queue there
+        cost a 4096^2 layer's RigL step 2%)."""
+        raw = _raw_stream(self.device.index)
+        if raw in self.joined:
             return
-        stream = torch.cuda.current_stream(self.arrays[0].device)
-        stream.wait_event(self.event)
+        stream = torch.cuda.current_stream(self.device)
+        build = torch.cuda.ExternalStream(self.stream, device=self.device)
+        stream.wait_event(build.record_event())
         for a in self.arrays:
             a.record_stream(stream)
+        self.joined.add(raw)
 
 
 # A row is "heavy" for slk_spmm's LDS-staged kernel when it holds more than
@@ -291,7 +304,12 @@ class PaddedCSR:
         msg = self._check()
         if msg:
             raise ValueError("PaddedCSR invariant check failed: " + msg)
-        self._nnz = int(nz.to(torch.int64).sum().item()) if nrows else 0
+        if self._on_device() and 0 < nrows < self._ORDER_MIN_ROWS:
+            host = nz.cpu().numpy()  # (one read serves both)
+            self._nnz = int(host.sum(dtype=np.int64))
+            self._heavy_hint = heavy_row_count(host)
+        else:
+            self._nnz = int(nz.to(torch.int64).sum().item()) if nrows else 0
 
     # internal constructor: trusted arrays (kernel outputs), no validation
     @classmethod
@@ -325,7 +343,7 @@ class PaddedCSR:
         self._seglist = None
         self._phased = None
         self._binned = None
-        self._strip_sizes = (-1, {})  # topology_version, N: the strips' sizes, or None
+        self._strip_choices = {}  # see _strip_choice
         # topology_version and what graphs captured under it read (see _pin)
         self._pinned = (-1, [])
         # True when a few columns hold many of the slots (a transpose of a
@@ -456,10 +474,10 @@ class PaddedCSR:
             return v
         if torch.cuda.is_current_stream_capturing():
             self._pin(built)
-        elif _lib.stream_of(self._col) == built.stream:
-            return v
-        else:
+        elif built.elsewhere():
             built.join()
+        else:
+            return v
         if v.n_dense_rows:  # the kept scratch belongs to calls on the build's stream
             own = self._dense_scratch(v.n_dense_rows)
             v = self._derived(v, dense_ws=_lib.ptr(own))
@@ -644,21 +662,18 @@ class PaddedCSR:
 
         return self._kept("_strips_kept", tuple(sizes), build, recorded=True)
 
-    # Strip choices kept per topology, by N.
-    _KEEP = 4
-
     def _strip_choice(self, N: int):
         """Sizes of the strips that dW should run with at N columns, None for
-        slk_sddmm (slk_strip_choose; host arithmetic of some 10 us, so kept)."""
-        version, kept = self._strip_sizes
-        if version != self._topology_version:
-            kept = {}
-            self._strip_sizes = (self._topology_version, kept)
-        if N not in kept:
-            while len(kept) >= self._KEEP:
-                kept.pop(next(iter(kept)), None)
-            kept[N] = _lib.strip_choose(self._view(), int(N))[0]
-        return kept[N]
+        slk_sddmm (slk_strip_choose). Some 4 us of host arithmetic on shape,
+        capacity, N and the counts of heavy and dense rows, so kept by what of
+        that can change."""
+        view, kept = self._view(), self._strip_choices
+        key = (int(N), view.n_heavy_rows, view.n_dense_rows)
+        if key not in kept:
+            if len(kept) >= 64:
+                kept.clear()
+            kept[key] = _lib.strip_choose(view, key[0])[0]
+        return kept[key]
 
     def _rows_host(self):
         h = self._host_rows

@@ -217,10 +217,8 @@ _CAPTURED_MIN_WORK_ALIGNED = 3_000_000_000
 
 
 def _recording_pays(W: PaddedCSR, N: int) -> bool:
-    """False where this call is captured and the build of quads or strips, run
-    by every replay, would cost more than they gain."""
-    return not torch.cuda.is_current_stream_capturing() or \
-        W.nnz * N >= (_CAPTURED_MIN_WORK if N % 4 else _CAPTURED_MIN_WORK_ALIGNED)
+    """Whether a captured call gains by quads or strips that every replay builds."""
+    return W.nnz * N >= (_CAPTURED_MIN_WORK if N % 4 else _CAPTURED_MIN_WORK_ALIGNED)
 
 
 # The estimates behind quads and strips take rows of like length, and refuse
@@ -260,11 +258,13 @@ def _quad_halves(W: PaddedCSR, K: int, N: int) -> int:
     if W.nnz * N < _QUAD_MIN_WORK or "bin_shape" in _overrides or "spmm_phases" in _overrides:
         return 0
     halves = _lib.quad_halves(W._view(), N)
-    if not halves or not _recording_pays(W, N) or _skew_slows_quads(W, N):
+    if not halves or _skew_slows_quads(W, N):
         return 0
-    if torch.cuda.is_current_stream_capturing() and \
-            _lib.quad_bytes(W._view(), halves) > _lib.QUAD_READ_BYTES:
-        return 0  # a graph cannot read their exact size, and would hold the bound
+    # (a graph cannot read the exact size of large quads, and would hold the bound)
+    if torch.cuda.is_current_stream_capturing() and (
+            not _recording_pays(W, N) or
+            _lib.quad_bytes(W._view(), halves) > _lib.QUAD_READ_BYTES):
+        return 0
     return halves
 
 
@@ -380,7 +380,11 @@ def _strip_sizes(W: PaddedCSR, N: int):
             not _lib.FORCED_KNOBS.isdisjoint(("sddmm_g", "seg_lean", "seg_group")):
         return None
     sizes = W._strip_choice(N)
-    return sizes if sizes and _recording_pays(W, N) and not _skew_slows_strips(W, N) else None
+    if not sizes or _skew_slows_strips(W, N):
+        return None
+    if torch.cuda.is_current_stream_capturing() and not _recording_pays(W, N):
+        return None
+    return sizes
 
 
 def _launch_sddmm(W: PaddedCSR, dY: torch.Tensor, X: torch.Tensor, kernel: str,
