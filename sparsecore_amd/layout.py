@@ -645,12 +645,17 @@ class PaddedCSR:
         values. With perm (this matrix is a transpose, perm its slot map) the
         slots are those of the matrix it was built from. Under graph capture the
         build is recorded with the call, so that a replay follows the rows as
-        they are."""
+        they are; a transpose's rows never change, so its quads are pinned."""
         def build():
             q = _lib.quad_build(self._view(), perm, int(halves), self.device)
             return q, q.arrays
 
-        return self._kept("_quads_kept", (int(halves), perm is not None), build, recorded=True)
+        return self._kept("_quads_kept", (int(halves), perm is not None), build,
+                          recorded=perm is None)
+
+    def _has_quads(self, halves: int, mapped: bool) -> bool:
+        version, kept = self._quads_kept
+        return version == self._topology_version and (halves, mapped) in kept
 
     def _strips(self, sizes) -> _lib.StripView:
         """The dW strips of slk_sddmm_strips for sizes (block, slots, per_wave,

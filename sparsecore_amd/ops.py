@@ -249,9 +249,9 @@ def _skew_slows_strips(W: PaddedCSR, N: int) -> bool:
     return (N % 4 == 0 or W.nnz * N < _SKEW_STRIP_MIN_WORK) and _skewed(W)
 
 
-def _quad_halves(W: PaddedCSR, K: int, N: int) -> int:
+def _quad_halves(W: PaddedCSR, K: int, N: int, mapped: bool = False) -> int:
     """64-column halves of the row quads (1 or 2) to run W on a K x N X with;
-    0: slk_spmm."""
+    0: slk_spmm. mapped: W is a cached transpose, run through its slot map."""
     forced = _overrides.get("quad")
     if forced is not None:
         return int(forced)
@@ -261,9 +261,9 @@ def _quad_halves(W: PaddedCSR, K: int, N: int) -> int:
     if not halves or _skew_slows_quads(W, N):
         return 0
     # (a graph cannot read the exact size of large quads, and would hold the bound)
-    if torch.cuda.is_current_stream_capturing() and (
-            not _recording_pays(W, N) or
-            _lib.quad_bytes(W._view(), halves) > _lib.QUAD_READ_BYTES):
+    if torch.cuda.is_current_stream_capturing() and not (mapped and W._has_quads(halves, True)) \
+            and (not _recording_pays(W, N) or
+                 _lib.quad_bytes(W._view(), halves) > _lib.QUAD_READ_BYTES):
         return 0
     return halves
 
@@ -482,7 +482,7 @@ def _spmm_backward(W: PaddedCSR, X: torch.Tensor, dY_f32: torch.Tensor, kernel: 
         dW_values = _launch_sddmm(W, dY_f32, _device_f32(X), kernel, dbias)
     if need_dx:
         WT, perm, fresh = _transpose_entry(W)
-        halves = _quad_halves(WT, *dY_f32.shape)
+        halves = _quad_halves(WT, *dY_f32.shape, mapped=True)
         if halves:  # through W's values: no refresh of WT's
             dX = torch.empty((W.ncols, dY_f32.shape[1]), dtype=torch.float32, device=W.device)
         if not halves or not _spmm_quads(WT, W.values, dY_f32, dX, halves, perm):

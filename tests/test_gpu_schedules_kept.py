@@ -96,3 +96,42 @@ def test_replay_after_warm_up_other_sizes_and_a_rewritten_row(dev, monkeypatch, 
         n = 115 - 20 * step
         W.rewrite_row(7 + step, list(range(step, step + n)), np.full(n, 0.5, np.float32))
         run(W, X, dY)
+
+
+def test_captured_input_gradient_keeps_its_transposes_quads(dev, monkeypatch):
+    """dX captured after warm-up runs on the quads kept with the cached transpose,
+    and replays right after eager calls of other sizes; once the matrix has a new
+    topology, a replay still reads the pinned ones (old rows, new values)."""
+    monkeypatch.setitem(ops._overrides, "quad", 1)
+    c = oracle.uniform_rows(300, 270, 40, seed=7, sigma=1.0)
+    W = from_oracle(c, dev)
+    X, dY = _t((270, 100), dev, 8), _t((300, 100), dev, 9)
+    run = lambda n=None: ops._spmm_backward(W, X, dY if n is None else _t((300, n), dev, n),
+                                            "simd", False, True)[1]
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        for _ in range(3):
+            run()
+    torch.cuda.current_stream().wait_stream(side)
+    WT = ops._transpose_entry(W)[0]
+    assert WT._has_quads(1, True)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        dX = run()
+    assert len(WT._pinned[1]) == 1 and W._pinned[1][0][2] is WT
+    for step in range(3):
+        for n in (64, 333, 1001):
+            run(n)
+        W.values.mul_(-2.0)
+        graph.replay()
+        torch.cuda.synchronize()
+        want = run()
+        assert_bits_equal(dX.cpu().numpy(), want.cpu().numpy(), f"replay {step}")
+    del WT
+    W.rewrite_row(0, [1, 2], [0.0, 0.0])
+    assert ops._transpose_entry(W)[0] is not W._pinned[1][0][2]
+    torch.empty(1 << 22, device=dev).fill_(float("nan"))
+    graph.replay()
+    torch.cuda.synchronize()
+    assert torch.isfinite(dX).all()
