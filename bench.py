@@ -119,6 +119,39 @@ def flops(nnz, N):
     return 2 * nnz * N
 
 
+# ───────────────────── the path's kernels, as ops runs them ───────────────────
+
+def dx_through_slot_map(WT, dY) -> bool:
+    """Whether dX = WT·dY reads W's values through the transpose's slot map (row
+    quads), with no refresh of WT's."""
+    from sparsecore_amd import ops
+
+    return ops._quad_halves(WT, *dY.shape, mapped=True) > 0
+
+
+def path_kernels(W, X, dY, tag, dx_tag):
+    """(label, call, bytes, flops) of the forward, dW and (dx_tag not None) dX of W
+    as the step launches them: ops chooses quads, strips and schedules. Where dX
+    needs the transpose's values refreshed, that is a label of its own."""
+    from sparsecore_amd import _lib, ops
+
+    (M, K), N = W.shape, X.shape[1]
+    out = [(f"spmm_fwd{tag}", lambda: ops._launch_spmm(W, X), bytes_fwd(W.nnz, M, K, N),
+            flops(W.nnz, N)),
+           (f"sddmm_dw{tag}", lambda: ops._launch_sddmm(W, dY, X, "simd"),
+            bytes_dw(W.nnz, W.total_capacity, M, K, N), flops(W.nnz, N))]
+    if dx_tag is None:
+        return out
+    WT, perm = ops._cached_transpose(W), ops._transpose_cache[id(W)][3]
+    dx = (f"spmm_dx{dx_tag}", lambda: ops._launch_spmm(WT, dY, halves=0), bytes_fwd(W.nnz, K, M, N),
+          flops(W.nnz, N))
+    if dx_through_slot_map(WT, dY):
+        return out + [dx[:1] + (lambda: ops._spmm_backward(W, X, dY, "simd", False, True),) + dx[2:]]
+    return out + [(f"transpose_refresh{tag}",
+                   lambda: _lib.transpose_refresh(W.values, perm, WT.values),
+                   bytes_refresh(W.nnz, WT.total_capacity), 0), dx]
+
+
 # ───────────────────────────── timing helpers ────────────────────────────────
 
 KERNEL_WARMUP = 3
@@ -323,27 +356,9 @@ class C2:
                             bytes_dw(W.nnz, W.total_capacity, M, K, N) +
                             bytes_fwd(W.nnz, K, M, N), 2 * flops(W.nnz, N)))
                 continue
-            Y = torch.empty(M, N, device=self.dev)
-            dY = torch.randn(M, N, device=self.dev)
-            out.append((f"spmm_fwd[{tag} {M}x{K}]",
-                        lambda view=view, X=X, Y=Y: _lib.spmm(view, X, Y),
-                        bytes_fwd(W.nnz, M, K, N), flops(W.nnz, N)))
-            out.append((f"sddmm_dw[{tag} {M}x{K}]",
-                        lambda view=view, dY=dY, X=X, dW=dW: _lib.sddmm(view, dY, X, dW,
-                                                                       _lib.SLK_DW_SIMD),
-                        bytes_dw(W.nnz, W.total_capacity, M, K, N), flops(W.nnz, N)))
-            if tag == "l2":  # layer 1's input needs no gradient, so no dX there
-                WT = ops._cached_transpose(W)
-                perm = ops._transpose_cache[id(W)][3]
-                dX = torch.empty(K, N, device=self.dev)
-                vT = WT._view()
-                out.append((f"spmm_dx[{tag} {K}x{M}]",
-                            lambda vT=vT, dY=dY, dX=dX: _lib.spmm(vT, dY, dX),
-                            bytes_fwd(WT.nnz, K, M, N), flops(W.nnz, N)))
-                out.append((f"transpose_refresh[{tag}]",
-                            lambda W=W, perm=perm, WT=WT: _lib.transpose_refresh(
-                                W.values, perm, WT.values),
-                            bytes_refresh(W.nnz, WT.total_capacity), 0))
+            # (layer 1's input needs no gradient, so no dX there)
+            out += path_kernels(W, X, torch.randn(M, N, device=self.dev), f"[{tag} {M}x{K}]",
+                                f"[{tag} {K}x{M}]" if tag == "l2" else None)
         return out
 
     def spmm_layer(self):
@@ -469,28 +484,14 @@ class GPTWork:
         """The HIP kernels of block 0's four sparse layers at N = batch*ctx tokens."""
         import torch
 
-        from sparsecore_amd import _lib, ops
-
         N = self.batch * self.ctx
         out = []
         for tag, layer in self.sparse_layers():
             W = layer._csr
             M, K = W.nrows, W.ncols
-            X = torch.randn(K, N, device=self.dev)
-            Y = torch.empty(M, N, device=self.dev)
-            dY = torch.randn(M, N, device=self.dev)
-            dW = torch.empty(W.total_capacity, device=self.dev)
-            dX = torch.empty(K, N, device=self.dev)
-            WT = ops._cached_transpose(W)
-            v, vT = W._view(), WT._view()
-            out.append((f"spmm_fwd[{tag} {M}x{K}]", lambda v=v, X=X, Y=Y: _lib.spmm(v, X, Y),
-                        bytes_fwd(W.nnz, M, K, N), flops(W.nnz, N)))
-            out.append((f"sddmm_dw[{tag} {M}x{K}]",
-                        lambda W=W, dY=dY, X=X, dW=dW: _lib.sddmm(ops._sddmm_view(W, X), dY, X, dW,
-                                                                  _lib.SLK_DW_SIMD),
-                        bytes_dw(W.nnz, W.total_capacity, M, K, N), flops(W.nnz, N)))
-            out.append((f"spmm_dx[{tag} {K}x{M}]", lambda vT=vT, dY=dY, dX=dX: _lib.spmm(vT, dY, dX),
-                        bytes_fwd(W.nnz, K, M, N), flops(W.nnz, N)))
+            out += path_kernels(W, torch.randn(K, N, device=self.dev),
+                                torch.randn(M, N, device=self.dev), f"[{tag} {M}x{K}]",
+                                f"[{tag} {K}x{M}]")
         return out
 
     def spmm_layer(self):
@@ -670,8 +671,9 @@ class LayerWork:
         if self.fused():
             return bytes_fwd(W.nnz, M, K, N) + bytes_backward_fused(W.nnz, W.total_capacity,
                                                                     M, K, N)
+        refresh = 0 if dx_through_slot_map(WT, self.dY) else bytes_refresh(W.nnz, WT.total_capacity)
         return (bytes_fwd(W.nnz, M, K, N) + bytes_dw(W.nnz, W.total_capacity, M, K, N)
-                + bytes_refresh(W.nnz, WT.total_capacity) + bytes_fwd(W.nnz, K, M, N))
+                + refresh + bytes_fwd(W.nnz, K, M, N))
 
     def step_flops(self):
         return 3 * flops(self.W.nnz, self.N)
@@ -683,32 +685,17 @@ class LayerWork:
 
         W = self.W
         M, K, N = self.M, self.K, self.N
-        WT = self._WT()
-        perm = ops._transpose_cache[id(W)][3]
-        Y = torch.empty(M, N, device=self.dev)
-        dW = torch.empty(W.total_capacity, device=self.dev)
-        dX = torch.empty(K, N, device=self.dev)
-        v, vT = ops._spmm_view(W, self.X), ops._spmm_view(WT, self.dY)
         if self.fused():
             WTs, perm_s = ops._cached_transpose_structure(W)
-            return [
-                ("spmm_fwd", lambda: _lib.spmm(v, self.X, Y), bytes_fwd(W.nnz, M, K, N),
-                 flops(W.nnz, N)),
+            dW = torch.empty(W.total_capacity, device=self.dev)
+            dX = torch.empty(K, N, device=self.dev)
+            return path_kernels(W, self.X, self.dY, "", None)[:1] + [
                 ("backward_fused", lambda: _lib.backward_fused(W._view(), WTs._view(), perm_s,
                                                                self.dY, self.X, dW, None, dX),
                  bytes_backward_fused(W.nnz, W.total_capacity, M, K, N), 2 * flops(W.nnz, N)),
             ] + (self._rigl_kernels() if self.rigl else [])
-        return [
-            ("spmm_fwd", lambda: _lib.spmm(v, self.X, Y), bytes_fwd(W.nnz, M, K, N),
-             flops(W.nnz, N)),
-            ("sddmm_dw", lambda: _lib.sddmm(ops._sddmm_view(W, self.X), self.dY, self.X, dW,
-                                            _lib.SLK_DW_SIMD),
-             bytes_dw(W.nnz, W.total_capacity, M, K, N), flops(W.nnz, N)),
-            ("transpose_refresh", lambda: _lib.transpose_refresh(W.values, perm, WT.values),
-             bytes_refresh(W.nnz, WT.total_capacity), 0),
-            ("spmm_dx", lambda: _lib.spmm(vT, self.dY, dX), bytes_fwd(W.nnz, K, M, N),
-             flops(W.nnz, N)),
-        ] + (self._rigl_kernels() if self.rigl else [])
+        return path_kernels(W, self.X, self.dY, "", "") + \
+            (self._rigl_kernels() if self.rigl else [])
 
     def _rigl_kernels(self):
         import torch
