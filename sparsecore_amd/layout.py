@@ -638,26 +638,22 @@ class PaddedCSR:
             c = self._binned = ((first, int(rw), int(h)), base, view, arrays)
         return c[2]
 
-    def _quads(self, halves: int, perm: torch.Tensor | None = None) -> _lib.QuadView:
+    def _quads(self, halves: int, perm: torch.Tensor | None = None,
+               recorded: bool = False) -> _lib.QuadView:
         """The row quads of slk_spmm_quad for 64·halves columns a row, built on
-        the device (slk_quad_build, three launches, no host read) once per
-        topology. They list slots, not values, so they survive a change of
-        values. With perm (this matrix is a transpose, perm its slot map) the
-        slots are those of the matrix it was built from. Under graph capture the
-        build is recorded with the call, so that a replay follows the rows as
-        they are; a transpose's rows never change, so its quads are pinned."""
+        the device (slk_quad_build, three launches; large ones with a host read)
+        once per topology. They list slots, not values, so they survive a change
+        of values. With perm (this matrix is a transpose, perm its slot map) the
+        slots are those of the matrix it was built from. recorded: under graph
+        capture the build is recorded with the call, so that a replay follows the
+        rows as they are."""
         def build():
             q = _lib.quad_build(self._view(), perm, int(halves), self.device)
             return q, q.arrays
 
-        return self._kept("_quads_kept", (int(halves), perm is not None), build,
-                          recorded=perm is None)
+        return self._kept("_quads_kept", (int(halves), perm is not None), build, recorded)
 
-    def _has_quads(self, halves: int, mapped: bool) -> bool:
-        version, kept = self._quads_kept
-        return version == self._topology_version and (halves, mapped) in kept
-
-    def _strips(self, sizes) -> _lib.StripView:
+    def _strips(self, sizes, recorded: bool = False) -> _lib.StripView:
         """The dW strips of slk_sddmm_strips for sizes (block, slots, per_wave,
         parts), built on the device (slk_strip_build, three launches, no host
         read) and kept, or recorded, like the quads."""
@@ -665,7 +661,11 @@ class PaddedCSR:
             t = _lib.strip_build(self._view(), 0, False, *sizes, self.device)
             return t, t.arrays
 
-        return self._kept("_strips_kept", tuple(sizes), build, recorded=True)
+        return self._kept("_strips_kept", tuple(sizes), build, recorded)
+
+    def _has(self, name: str, key) -> bool:
+        version, kept = getattr(self, name)
+        return version == self._topology_version and key in kept
 
     def _strip_choice(self, N: int):
         """Sizes of the strips that dW should run with at N columns, None for

@@ -204,15 +204,18 @@ _overrides: dict[str, object] = {}
 # that does, 1152 x 384 at 10% and N = 1001, has 4.4e7), so the call is spared.
 _QUAD_MIN_WORK = 30_000_000
 
-# Under graph capture a call records the build of its quads or strips with
-# itself, so that a replay follows the rows as they are and the graph owns all
+# Under graph capture a call whose plain kernel reads nothing but the matrix's own
+# arrays records the build of its quads or strips with itself, so that a replay
+# follows the rows as they are, as the plain kernel's would, and the graph owns all
 # that it reads. The build adds 9-20 us to each replay (4096 x 1024 to 4096^2 at
 # 30% the most), which they repay from this many live slots x N on: where N is
 # not a multiple of 4 (1152 x 384 at 30%, N = 1001: forward 49 -> 44 us, dW 42 ->
 # 40; 2304 x 768 at 30%, N = 1001: 161 -> 74, 145 -> 65; 4096 x 1024 at 10%, N =
 # 333, below the line: dW 53 -> 57) and where it is (2304 x 768 at 30%, N = 8192:
-# 289 -> 269, 367 -> 300; 3072 x 768 at 30%, N = 2048, below: 107 -> 109).
-_CAPTURED_MIN_WORK = 200_000_000
+# forward 289 -> 269; 3072 x 768 at 30%, N = 2048, below: 107 -> 109). Where the
+# plain kernel needs a schedule of the topology itself, as the segment kernel does,
+# a captured call runs on the quads or strips that its warm-up kept.
+_CAPTURED_MIN_WORK = 150_000_000
 _CAPTURED_MIN_WORK_ALIGNED = 3_000_000_000
 
 
@@ -260,11 +263,12 @@ def _quad_halves(W: PaddedCSR, K: int, N: int, mapped: bool = False) -> int:
     halves = _lib.quad_halves(W._view(), N)
     if not halves or _skew_slows_quads(W, N):
         return 0
-    # (a graph cannot read the exact size of large quads, and would hold the bound)
-    if torch.cuda.is_current_stream_capturing() and not (mapped and W._has_quads(halves, True)) \
-            and (not _recording_pays(W, N) or
-                 _lib.quad_bytes(W._view(), halves) > _lib.QUAD_READ_BYTES):
-        return 0
+    if torch.cuda.is_current_stream_capturing():
+        if mapped or _spmm_scheduled(W, K, N):
+            return halves if W._has("_quads_kept", (halves, mapped)) else 0
+        # (a graph cannot read the exact size of large quads, and would hold the bound)
+        if not _recording_pays(W, N) or _lib.quad_bytes(W._view(), halves) > _lib.QUAD_READ_BYTES:
+            return 0
     return halves
 
 
@@ -274,18 +278,31 @@ def _spmm_quads(W: PaddedCSR, values: torch.Tensor, X: torch.Tensor, Y: torch.Te
     """Y = W·X (+ bias) through W's row quads. False, with nothing launched and
     W's quads given up, where the memory for them is not to be had: slk_spmm needs
     none."""
+    recorded = perm is None and not _spmm_scheduled(W, *X.shape)
     try:
-        _lib.spmm_quad(W._view(), W._quads(halves, perm), values, X, Y, bias)
+        _lib.spmm_quad(W._view(), W._quads(halves, perm, recorded), values, X, Y, bias)
     except torch.OutOfMemoryError:
         W._quads_kept = (-1, {})
         return False
     return True
 
 
+def _phases(W: PaddedCSR, K: int, N: int) -> int:
+    """Column phases of slk_spmm's gather path where X is far beyond the L2s and
+    W's columns are not skewed; 0: one sweep."""
+    if 4 * K * N >= _PHASE_MIN_X_BYTES and K > _PHASE_X_ROWS and not W._cols_skewed:
+        return -(-K // _PHASE_X_ROWS)
+    return 0
+
+
+def _spmm_scheduled(W: PaddedCSR, K: int, N: int) -> bool:
+    """Whether slk_spmm would run W by a schedule of its topology."""
+    return _phases(W, K, N) > 0 or _bin_shape(W, K, N) is not None
+
+
 def _spmm_view(W: PaddedCSR, X: torch.Tensor):
     """W's view for slk_spmm: with a binned slot stream where it pays (see
-    above), else with phase bounds where X is far beyond the L2s and W's
-    columns are not skewed."""
+    above), else with phase bounds."""
     K, N = X.shape
     binned = _overrides.get("bin_shape")
     if binned is None:
@@ -293,11 +310,8 @@ def _spmm_view(W: PaddedCSR, X: torch.Tensor):
     if binned:
         return W._view_binned(*binned)
     forced = _overrides.get("spmm_phases")
-    if forced is not None:
-        return W._view_phased(int(forced)) if int(forced) > 1 else W._view()
-    if 4 * K * N >= _PHASE_MIN_X_BYTES and K > _PHASE_X_ROWS and not W._cols_skewed:
-        return W._view_phased(-(-K // _PHASE_X_ROWS))
-    return W._view()
+    phases = _phases(W, K, N) if forced is None else int(forced)
+    return W._view_phased(phases) if phases > 1 else W._view()
 
 
 def _launch_spmm(W: PaddedCSR, X: torch.Tensor, bias: torch.Tensor | None = None,
@@ -357,9 +371,14 @@ def _sddmm_view(W: PaddedCSR, X: torch.Tensor):
     forced = _overrides.get("seg")
     if forced is not None:
         return W._view_segmented(*forced, skip_dense=skip) if forced else W._view()
-    if W.nnz >= _SEG_MIN_NNZ and N >= 1024 and N % 4 == 0:
+    if _sddmm_scheduled(W, N):
         return W._view_segmented(*_seg_shape(W, K, N), skip_dense=skip)
     return W._view()
+
+
+def _sddmm_scheduled(W: PaddedCSR, N: int) -> bool:
+    """Whether slk_sddmm would run W by a segment list."""
+    return W.nnz >= _SEG_MIN_NNZ and N >= 1024 and N % 4 == 0
 
 
 # Strips (slk_sddmm_strips) instead of slk_sddmm where slk_strip_choose expects
@@ -382,8 +401,9 @@ def _strip_sizes(W: PaddedCSR, N: int):
     sizes = W._strip_choice(N)
     if not sizes or _skew_slows_strips(W, N):
         return None
-    if torch.cuda.is_current_stream_capturing() and not _recording_pays(W, N):
-        return None
+    if torch.cuda.is_current_stream_capturing():
+        if not (W._has("_strips_kept", sizes) if _sddmm_scheduled(W, N) else _recording_pays(W, N)):
+            return None
     return sizes
 
 
@@ -394,7 +414,8 @@ def _launch_sddmm(W: PaddedCSR, dY: torch.Tensor, X: torch.Tensor, kernel: str,
     sizes = _strip_sizes(W, X.shape[1]) if order == _lib.SLK_DW_SIMD else None
     if sizes:
         try:
-            _lib.sddmm_strips(W._view(), W._strips(sizes), dY, X, dW, dbias)
+            strips = W._strips(sizes, not _sddmm_scheduled(W, X.shape[1]))
+            _lib.sddmm_strips(W._view(), strips, dY, X, dW, dbias)
             return dW
         except torch.OutOfMemoryError:  # for the strips or their copy of X
             W._strips_kept = (-1, {})

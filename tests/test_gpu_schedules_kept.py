@@ -115,7 +115,7 @@ def test_captured_input_gradient_keeps_its_transposes_quads(dev, monkeypatch):
             run()
     torch.cuda.current_stream().wait_stream(side)
     WT = ops._transpose_entry(W)[0]
-    assert WT._has_quads(1, True)
+    assert WT._has("_quads_kept", (1, True))
     graph = torch.cuda.CUDAGraph()
     with torch.cuda.graph(graph):
         dX = run()

@@ -59,8 +59,8 @@ def test_a_refused_value_buffer_gives_the_kept_quads_up(calls, monkeypatch):
 
 
 def test_large_quads_are_not_recorded_in_graphs(monkeypatch):
-    v = _lib.CsrView(16384, 16384, int(1.2 * 0.05 * 16384 ** 2), 8, 8, 8, 8, 8)
-    assert _lib.quad_halves(v, 4096) > 0 and _lib.quad_bytes(v, 1) > _lib.QUAD_READ_BYTES
+    v = _lib.CsrView(200000, 4096, int(1.2 * 0.05 * 200000 * 4096), 8, 8, 8, 8, 8)
+    assert _lib.quad_halves(v, 8192) > 0 and _lib.quad_bytes(v, 1) > _lib.QUAD_READ_BYTES
     small = _lib.CsrView(2304, 768, int(1.2 * 0.3 * 2304 * 768), 8, 8, 8, 8, 8)
     assert _lib.quad_bytes(small, 1) < _lib.QUAD_READ_BYTES
     W = from_oracle(oracle.uniform_rows(16, 16, 2, seed=1))
