@@ -524,7 +524,7 @@ extern "C" int64_t slk_quad_halves(const slk_csr* W, int64_t N) {
     double least = 0.0;
     int best = 0;
     for (const int h : {1, 2}) {
-        if (slk_quad_chunks(W->ncols, h) > kMaxChunks) continue;
+        if (slk_quad_chunks(W->ncols, h) > kMaxChunks || slk_quad_windows(W, h) > INT32_MAX) continue;
         double c;
         quad_rw(W, h, N, &c);
         if (best == 0 || c < least) {
@@ -549,7 +549,8 @@ int quad_extent(const slk_csr* W, int64_t halves, int64_t ws_words, const char* 
     *nq = ceil_div(W->nrows, int64_t{4});
     *nch = slk_quad_chunks(W->ncols, halves);
     if (*nch > kMaxChunks) return fail(SLK_EINVAL, at + "too many columns");
-    if (*nq > INT32_MAX) return fail(SLK_EINVAL, at + "too many rows");
+    if (*nq > INT32_MAX || slk_quad_windows(W, halves) > INT32_MAX)  // (their scan is 32-bit)
+        return fail(SLK_EINVAL, at + "too many windows");
     const int64_t need = *nq * 4 * (*nch + 1);
     if (ws_words < need)
         return fail(SLK_EINVAL, at + "workspace of " + std::to_string(ws_words) + " words, needs " +
@@ -584,8 +585,7 @@ extern "C" int slk_quad_fill(const slk_csr* W, const int64_t* perm, int64_t halv
     using namespace slk;
     int64_t nq = 0, nch = 0;
     if (int rc = quad_extent(W, halves, ws_words, "quad_build", &nq, &nch)) return rc;
-    if (n_windows < 1 || n_windows > INT32_MAX)
-        return fail(SLK_EINVAL, "quad_build: no or too many windows");
+    if (n_windows < 1) return fail(SLK_EINVAL, "quad_build: no windows");
     if (ws == nullptr || start == nullptr || count == nullptr || offset == nullptr ||
         slot == nullptr || used == nullptr)
         return fail(SLK_EINVAL, "quad_build: NULL output");
@@ -607,7 +607,6 @@ extern "C" int slk_quad_build(const slk_csr* W, const int64_t* perm, int64_t hal
         return fail(SLK_EINVAL, "quad_build: workspace of " + std::to_string(n_windows) +
                                     " windows, needs " +
                                     std::to_string(slk_quad_windows(W, halves)));
-    if (n_windows > INT32_MAX) return fail(SLK_EINVAL, "quad_build: too many windows");
     if (offset == nullptr || slot == nullptr) return fail(SLK_EINVAL, "quad_build: NULL output");
     if (int rc = slk_quad_count(W, halves, ws, ws_words, start, count, used, stream)) return rc;
     return slk_quad_fill(W, perm, halves, ws, ws_words, start, count, offset, slot, n_windows, used,

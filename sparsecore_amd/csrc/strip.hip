@@ -36,6 +36,7 @@ namespace {
 constexpr uint32_t kBufWord3 = 0x00020000;  // gfx9 buffer resource dword 3
 constexpr int kWin = 64;                    // columns of N per (part of a) window
 constexpr int64_t kMaxBlocks = 2048;
+constexpr int64_t kMaxRows = int64_t{4} * 256 * 65535;  // the fill's grid is 256 quads per row of blocks
 
 constexpr int kWaves = 16;
 constexpr int kMaxC = 256;                  // X rows per block
@@ -439,6 +440,7 @@ int check_strips(const slk_csr* W, const slk_strips* T, const char* who) {
     if (T->block < 16 || T->block > kMaxC || T->block % 16 != 0)
         return fail(SLK_EINVAL, at + "blocks are multiples of 16 up to 256 columns");
     if (ceil_div(W->ncols, T->block) > kMaxBlocks) return fail(SLK_EINVAL, at + "too many columns");
+    if (W->nrows > kMaxRows) return fail(SLK_EINVAL, at + "too many rows");
     if ((T->first > 0 || T->ordered != 0) && W->row_order == nullptr)
         return fail(SLK_EINVAL, at + "no row order");
     if (T->slots < 1 || T->slots > 128 || T->per_wave < 1 || T->per_wave > 8)
@@ -530,7 +532,8 @@ extern "C" int slk_strip_choose(const slk_csr* W, int64_t N, slk_strips* T, doub
     if (T == nullptr || us == nullptr) return fail(SLK_EINVAL, "strip_choose: NULL output");
     *T = slk_strips{};
     *us = 0.0;
-    if (W->nrows == 0 || W->ncols == 0 || N < 1 || N > (int64_t{1} << 21)) return SLK_OK;
+    if (W->nrows == 0 || W->nrows > kMaxRows || W->ncols == 0 || N < 1 || N > (int64_t{1} << 21))
+        return SLK_OK;
     // rows of very different lengths pad each other (16384^2 Zipf(1.1) at 95%:
     // 5.34 ms against 5.29, at 99% 3.3 against 2.1), and dense rows run on the
     // matrix cores
@@ -580,7 +583,6 @@ extern "C" int slk_strip_build(const slk_csr* W, const slk_strips* T, int32_t* i
     if (items == nullptr || rel == nullptr || used == nullptr || ws == nullptr)
         return fail(SLK_EINVAL, "strip_build: NULL output");
     const Extent e = strip_extent(W, T);
-    if (e.nq > INT32_MAX) return fail(SLK_EINVAL, "strip_build: too many rows");
     hipStream_t st = as_stream(stream);
     int32_t* total = ws + e.nb * e.nq;
     hipLaunchKernelGGL(strip_count_kernel, dim3(static_cast<unsigned>(e.nq)), dim3(256),

@@ -71,3 +71,14 @@ def test_quad_entry_points_check_their_arguments():
     assert call(_lib.QuadView(), 300, 8) == _lib.SLK_EINVAL
     assert call(q, 299, 8) == _lib.SLK_EINVAL and "shape" in lib.slk_last_error().decode()
     assert call(q, 300, 3) == _lib.SLK_EINVAL and "N outside" in lib.slk_last_error().decode()
+
+
+def test_more_windows_than_their_scan_counts_are_refused():
+    lib = _lib.load()
+    v = _lib.CsrView(1 << 26, 65536, 31 << 26, 8, 8, 8, 8, 8)
+    assert lib.slk_quad_windows(ctypes.byref(v), 1) > 2 ** 31
+    assert _lib.quad_halves(v, 4095) == 0
+    rc = lib.slk_quad_count(ctypes.byref(v), 1, 8, 1 << 40, 8, 8, 8, None)
+    assert rc == _lib.SLK_EINVAL and "windows" in lib.slk_last_error().decode()
+    rc = lib.slk_quad_fill(ctypes.byref(v), None, 1, 8, 1 << 40, 8, 8, 8, 8, 64, 8, None)
+    assert rc == _lib.SLK_EINVAL and "windows" in lib.slk_last_error().decode()

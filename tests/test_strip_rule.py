@@ -83,3 +83,14 @@ def test_strip_entry_points_check_their_arguments():
     assert call(ok, 65, 16, need - 1) == _lib.SLK_EINVAL
     assert "workspace" in lib.slk_last_error().decode()
     assert call(ok, 65, 8, need) == _lib.SLK_EINVAL
+
+
+def test_more_rows_than_the_build_can_take_stay_with_slk_sddmm():
+    M = 4 * 256 * 65535
+    v = lambda m: _lib.CsrView(m, 64, 20 * m, 8, 8, 8, 8, 8)
+    words = (ctypes.c_int64 * 3)()
+    T = _lib.StripView(8, 8, 8, 0, 0, 48, 32, 1, 2)
+    assert _lib.load().slk_strip_words(ctypes.byref(v(M)), ctypes.byref(T), words) == _lib.SLK_OK
+    assert _lib.load().slk_strip_words(ctypes.byref(v(M + 1)), ctypes.byref(T), words) == _lib.SLK_EINVAL
+    assert _lib.strip_choose(v(1 << 20), 1001)[0] is not None
+    assert _lib.strip_choose(v(M + 1), 1001)[0] is None
