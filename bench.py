@@ -143,7 +143,7 @@ def path_kernels(W, X, dY, tag, dx_tag):
     if dx_tag is None:
         return out
     WT, perm = ops._cached_transpose(W), ops._transpose_cache[id(W)][3]
-    dx = (f"spmm_dx{dx_tag}", lambda: ops._launch_spmm(WT, dY, halves=0), bytes_fwd(W.nnz, K, M, N),
+    dx = (f"spmm_dx{dx_tag}", lambda: ops._launch_spmm(WT, dY, quads=False), bytes_fwd(W.nnz, K, M, N),
           flops(W.nnz, N))
     if dx_through_slot_map(WT, dY):
         return out + [dx[:1] + (lambda: ops._spmm_backward(W, X, dY, "simd", False, True),) + dx[2:]]

@@ -17,17 +17,20 @@
 // contiguous bytes per row, conflict-free), one move for the value, and the
 // fmas: no readlane, no per-slot scalar work, and a branch every two steps.
 // Straight-line, that runs at 54 (64 columns a row) and 64 (128 columns)
-// TFLOP/s, bound by the vector unit's issue and the LDS reads. Rows of a quad
-// with fewer slots than its longest are padded with a zero X row and the value
+// TFLOP/s. What bounds it is the vector unit's issue: 2304 x 768 at 30%, N = 8192,
+// and the 16384^2 transpose at 5% keep it busy 74% and 73% of the cycles, with 8%
+// and 1% of the waves' cycles waiting to issue to the LDS; 6 to 8 instructions
+// per slot and 256 columns, padding included, of which the fmas are 4. Rows of a
+// quad with fewer slots than its longest are padded with a zero X row and the value
 // -0.0, which leaves every sum as it is (x + -0.0 = x for every x, NaN and
 // both zeros included).
 //
 // Measured against slk_spmm, values kernel included: 2304 x 768 at 20%, N =
-// 8192, 219 -> 169 us; 768 x 3072 at 30%, N = 4096, 265 -> 169; 4096^2 at 10%,
-// N = 4096, 540 -> 398 (34 TFLOP/s of useful slots; about a third of the
+// 8192, 238 -> 190 us; 768 x 3072 at 30%, N = 4096, 286 -> 196; 4096^2 at 10%,
+// N = 4096, 566 -> 462 (30 TFLOP/s of useful slots; about a third of the
 // steps are padding, the rest of the gap is the windows and chunk barriers);
-// 3072 x 768 at 10%, N = 1001, 82 -> 35 us (no 16-byte lanes: the other path
-// was the gather kernel).
+// 3072 x 768 at 10%, N = 1001, 87 -> 37 us (no 16-byte lanes: the other path
+// is the gather kernel).
 #include "common.hpp"
 
 namespace slk {
@@ -459,9 +462,10 @@ int launch_quad_rw(int rw, const slk_csr* W, const slk_quads* Q, const float* va
 // Estimated microseconds: rounds of workgroups (one per CU, by its LDS) x X
 // chunks x (staging and barrier + quads x (window + steps)), a step being one
 // slot of each of the quad's rows, as many per chunk as its longest row has
-// (about one standard deviation above the mean). Fitted to 109 layer shapes
-// (37 to 16384 rows, 50 to 4096 columns, N 41 to 16384, 1% to 60%) times every
-// configuration; the choice it gives is within 5% of the fastest on all of them.
+// (about one standard deviation above the mean). The constants are a fit to layer
+// shapes of 37 to 16384 rows, 50 to 4096 columns, N 41 to 16384 and 1% to 60%; of
+// the 524 shapes on which both sides are timed in profiles/schedule_choices.md
+// quads lose on two by over 3% (4% at most).
 double quad_cost(int64_t M, int64_t K, int64_t N, double density, int h, int rw) {
     const double mu = density * chunk_rows(h);
     const double steps = mu + 1.03 * __builtin_sqrt(mu) + 1.0;

@@ -1381,7 +1381,7 @@ int spmm_impl(const slk_csr* W, const float* X, int64_t K, int64_t N, const floa
 
 }  // namespace
 
-// Fitted like quad_cost, to the same 109 shapes: the LDS kernel 19.5 ns per
+// Fitted like quad_cost, to the same shapes: the LDS kernel 19.5 ns per
 // unit of lds_cost, the gather kernels the rate they reach once the slots
 // outweigh the launch (slots x columns per microsecond).
 double spmm_estimate(const slk_csr* W, int64_t N) {

@@ -19,12 +19,12 @@
 // once for all its slots of the strip, and each staged window serves the
 // workgroup's 64·R rows: 15-25 bytes from the L2 per slot and window, against
 // 50-64 for the segment kernel of sddmm.hip, whose quads of lanes take 8 slots
-// per dY read. What bounds it is the LDS: a 16-byte read per four fmas, 73
-// TFLOP/s of slots and padding at the 560 reads per us of a CU; it reaches about
-// two thirds of that (without the reads the fmas and offset adds alone take 170
-// of 254 us at 2304 x 768, 30%, N = 8192). Measured, layout and dbias included:
-// that layer 373 -> 280 us, 1152 x 384 at 30% 168 -> 118, 4096^2 at 5%, N =
-// 4096, 585 -> 380, 1537 x 1000 at 20%, N = 1777, 194 -> 56.
+// per dY read. What bounds it is the LDS, a 16-byte read per four fmas, beside
+// the vector unit: 73 TFLOP/s of slots and padding at the 560 reads per us of a CU,
+// of which it reaches about two thirds (2304 x 768 at 30%, N = 8192: vector unit
+// busy 57%, 24% of the waves' cycles waiting to issue to the LDS). Measured, layout
+// included: that layer 365 -> 283 us, 1152 x 384 at 30% 171 -> 125, 4096^2 at 5%,
+// N = 4096, 579 -> 405, 1537 x 1000 at 20%, N = 1777, 194 -> 52.
 #include "common.hpp"
 #include "dw_common.hpp"
 
@@ -471,8 +471,8 @@ int launch_strips(const slk_csr* W, const slk_strips* T, const float* dY, const 
     return check_launch("sddmm_strips");
 }
 
-// Estimated microseconds at N columns of strips of T's sizes (fitted to 105
-// layer shapes, 256 to 8192 rows, N 256 to 8192, 1% to 70%: rounds of
+// Estimated microseconds at N columns of strips of T's sizes (a fit to layer
+// shapes of 256 to 8192 rows, N 256 to 8192, 1% to 70%: rounds of
 // workgroups, one per CU, x windows x (barrier and staging + strips x (dY +
 // steps)), a step being one slot of each of a quad's rows, as many as the
 // longest row has), or a negative number where a row's slots of a block would
@@ -498,10 +498,10 @@ double strip_cost(int64_t M, int64_t K, int64_t N, double density, const slk_str
 // The same for slk_sddmm: what its kernels reach (slots x columns per ns), and
 // the chain of windows that one workgroup or wave runs however small the matrix.
 // Segment kernel: N % 4 == 0 and N >= 1024, from 100000 slots; 4-slot segments
-// below 1/16. The rates are those of 423 shapes on which both sides were timed
-// (256 to 4096 rows, 384 to 4096 columns, 3% to 30%, N 256 to 8192): strips then
-// lose by 11% at most (768 x 4096 at 5%, N = 2048: 59 -> 66 us) and by over 3% on
-// seven. From 1.5 million slots below 1/8 the segment kernel gains (4096^2 at 10%,
+// below 1/16. The rates are those of the shapes on which both sides are timed in
+// profiles/schedule_choices.md (256 to 4096 rows, 384 to 4096 columns, 3% to 30%, N
+// 256 to 8192): of 475 where strips are taken they lose by over 3% on six (10% at
+// most: 768 x 4096 at 5%, N = 2048, 58 -> 65 us). From 1.5 million slots below 1/8 the segment kernel gains (4096^2 at 10%,
 // N = 8192: 1254 us against 1402 in strips), as it does where rows hold over 40 of
 // 70000 to 100000 slots on the per-slot kernels (1000 x 768 at 10%, N = 1024: 19
 // against 23).

@@ -333,7 +333,7 @@ class PaddedCSR:
         self._cview = None
         # (topology_version, row order, heavy rows, dense rows, dense scratch, _Built)
         self._order = None
-        # schedules: topology_version, then by key a _Built (see _kept)
+        # schedules: topology_version, then by key a _Built (see _find)
         self._segs_kept = (-1, {})    # (block_cols, seg_slots, dense rows left out)
         self._phases_kept = (-1, {})  # n_phases
         self._bins_kept = (-1, {})    # (first, rw, h)
@@ -343,7 +343,6 @@ class PaddedCSR:
         self._seglist = None
         self._phased = None
         self._binned = None
-        self._strip_choices = {}  # see _strip_choice
         # topology_version and what graphs captured under it read (see _pin)
         self._pinned = (-1, [])
         # True when a few columns hold many of the slots (a transpose of a
@@ -463,7 +462,7 @@ class PaddedCSR:
                              _lib.ptr(self._row_nnz), _lib.ptr(self._row_cap), _lib.ptr(order),
                              n_heavy_rows=n_heavy, n_dense_rows=n_dense,
                              dense_ws=_lib.ptr(dws))
-            v.built = built
+            v.built, v.routes = built, {}
             if built is not None and torch.cuda.is_current_stream_capturing():
                 # an order that only the graph fills is the graph's alone
                 if self._order is None or self._order[5] is not built:
@@ -508,7 +507,7 @@ class PaddedCSR:
         fields = {f: getattr(base, f) for f, _ in _lib.CsrView._fields_}
         fields.update(changes)
         v = _lib.CsrView(**fields)
-        v.base = base  # and with it the arrays that only the base holds
+        v.base, v.routes = base, base.routes  # and the arrays that only the base holds
         return v
 
     # Lazily built device state (row order, schedules) is kept per topology. A
@@ -526,26 +525,30 @@ class PaddedCSR:
         if not any(p is held for p in pinned):
             pinned.append(held)
 
-    def _kept(self, name: str, key, build, recorded: bool = False):
-        """build()'s (value, arrays), kept under `key` for this topology; the
-        value. recorded: under capture always build anew, into the graph, whose
-        replays then follow the matrix's rows as they are."""
+    def _find(self, name: str, key, capturing: bool, recorded: bool = False):
+        """The value kept under `key` for this topology, ready for the current
+        stream; None where it has to be built: none is kept, or the call is
+        captured and recorded asks for a build in the graph, whose replays then
+        follow the matrix's rows as they are."""
         version, kept = getattr(self, name)
-        if version != self._topology_version:
-            kept = {}
-            setattr(self, name, (self._topology_version, kept))
-        capturing = torch.cuda.is_current_stream_capturing()
-        b = None if capturing and recorded else kept.get(key)
-        if b is None:
-            value, arrays = build()
-            if not capturing:
-                kept[key] = _Built(value, arrays)
-            return value
+        b = kept.get(key) if version == self._topology_version else None
+        if b is None or (capturing and recorded):
+            return None
         if capturing:
             self._pin(b)
         else:
             b.join()
         return b.value
+
+    def _keep(self, name: str, key, value, arrays, capturing: bool):
+        """value, just built into arrays, kept under `key`, unless by a capture."""
+        if not capturing:
+            version, kept = getattr(self, name)
+            if version != self._topology_version:
+                kept = {}
+                setattr(self, name, (self._topology_version, kept))
+            kept[key] = _Built(value, arrays)
+        return value
 
     def _view_segmented(self, block_cols: int, seg_slots: int,
                         skip_dense: bool = False) -> _lib.CsrView:
@@ -563,12 +566,12 @@ class PaddedCSR:
         skip = int(base.n_dense_rows) if skip_dense else 0
         key = (int(block_cols), int(seg_slots), skip)
 
-        def build():
+        capturing = torch.cuda.is_current_stream_capturing()
+        arrays = self._find("_segs_kept", key, capturing)
+        if arrays is None:
             arrays = _lib.seg_list_build(self._derived(base, seg_dense_rows=skip), key[0], key[1],
                                          self.device)
-            return arrays, arrays
-
-        arrays = self._kept("_segs_kept", key, build)
+            self._keep("_segs_kept", key, arrays, arrays, capturing)
         c = self._seglist
         if c is None or c[1] is not base or c[3] is not arrays:
             start, row, count, groups = arrays
@@ -588,11 +591,11 @@ class PaddedCSR:
         base = self._view()
         key = int(n_phases)
 
-        def build():
+        capturing = torch.cuda.is_current_stream_capturing()
+        lo = self._find("_phases_kept", key, capturing)
+        if lo is None:
             lo = _lib.phase_bounds_build(base, key, self.device)
-            return lo, (lo,)
-
-        lo = self._kept("_phases_kept", key, build)
+            self._keep("_phases_kept", key, lo, (lo,), capturing)
         c = self._phased
         if c is None or c[1] is not base or c[3] is not lo:
             view = self._derived(base, phase_lo=_lib.ptr(lo), n_phases=key)
@@ -622,12 +625,13 @@ class PaddedCSR:
         base view as the other schedules do."""
         base = self._view()
 
-        def build():
+        key = (int(base.n_heavy_rows), int(rw), int(h))
+        capturing = torch.cuda.is_current_stream_capturing()
+        kept = self._find("_bins_kept", key, capturing)
+        if kept is None:
             first, n_bin = self._bin_coverage()
             arrays = _lib.bin_build(base, first, int(rw), int(h), n_bin, self.device)
-            return (first, n_bin, arrays), arrays
-
-        kept = self._kept("_bins_kept", (int(base.n_heavy_rows), int(rw), int(h)), build)
+            kept = self._keep("_bins_kept", key, (first, n_bin, arrays), arrays, capturing)
         c = self._binned
         if c is None or c[1] is not base or c[3] is not kept[2]:
             first, n_bin, arrays = kept
@@ -638,47 +642,34 @@ class PaddedCSR:
             c = self._binned = ((first, int(rw), int(h)), base, view, arrays)
         return c[2]
 
-    def _quads(self, halves: int, perm: torch.Tensor | None = None,
+    def _quads(self, halves: int, perm: torch.Tensor | None = None, capturing: bool = False,
                recorded: bool = False) -> _lib.QuadView:
         """The row quads of slk_spmm_quad for 64·halves columns a row, built on
         the device (slk_quad_build, three launches; large ones with a host read)
         once per topology. They list slots, not values, so they survive a change
         of values. With perm (this matrix is a transpose, perm its slot map) the
-        slots are those of the matrix it was built from. recorded: under graph
-        capture the build is recorded with the call, so that a replay follows the
-        rows as they are."""
-        def build():
+        slots are those of the matrix it was built from. capturing, recorded: as
+        for _find."""
+        key = (halves, perm is not None)
+        q = self._find("_quads_kept", key, capturing, recorded)
+        if q is None:
             q = _lib.quad_build(self._view(), perm, int(halves), self.device)
-            return q, q.arrays
+            self._keep("_quads_kept", key, q, q.arrays, capturing)
+        return q
 
-        return self._kept("_quads_kept", (int(halves), perm is not None), build, recorded)
-
-    def _strips(self, sizes, recorded: bool = False) -> _lib.StripView:
+    def _strips(self, sizes, capturing: bool = False, recorded: bool = False) -> _lib.StripView:
         """The dW strips of slk_sddmm_strips for sizes (block, slots, per_wave,
         parts), built on the device (slk_strip_build, three launches, no host
         read) and kept, or recorded, like the quads."""
-        def build():
+        t = self._find("_strips_kept", sizes, capturing, recorded)
+        if t is None:
             t = _lib.strip_build(self._view(), 0, False, *sizes, self.device)
-            return t, t.arrays
-
-        return self._kept("_strips_kept", tuple(sizes), build, recorded)
+            self._keep("_strips_kept", sizes, t, t.arrays, capturing)
+        return t
 
     def _has(self, name: str, key) -> bool:
         version, kept = getattr(self, name)
         return version == self._topology_version and key in kept
-
-    def _strip_choice(self, N: int):
-        """Sizes of the strips that dW should run with at N columns, None for
-        slk_sddmm (slk_strip_choose). Some 4 us of host arithmetic on shape,
-        capacity, N and the counts of heavy and dense rows, so kept by what of
-        that can change."""
-        view, kept = self._view(), self._strip_choices
-        key = (int(N), view.n_heavy_rows, view.n_dense_rows)
-        if key not in kept:
-            if len(kept) >= 64:
-                kept.clear()
-            kept[key] = _lib.strip_choose(view, key[0])[0]
-        return kept[key]
 
     def _rows_host(self):
         h = self._host_rows

@@ -138,7 +138,10 @@ _PHASE_MIN_X_BYTES = 128 << 20
 _PHASE_X_ROWS = 4096
 
 
-# Binned slot stream for slk_spmm's LDS-staged kernel (slk_csr.bin_*): for
+# Binned slot stream for slk_spmm's LDS-staged kernel (slk_csr.bin_*). Row quads,
+# which are asked first, take nearly every shape that passes these bars (all but
+# 142 of 48987 sampled); what reaches it is the rest of them, captured calls whose
+# quads no warm-up kept, and calls that found no memory for quads. For
 # matrices without heavy rows where N is large, each staged X element is
 # expected to serve at least _BIN_MIN_REUSE rows of a workgroup (density x
 # rows per workgroup; fewer, and gathering X rows directly is faster), and a
@@ -199,8 +202,8 @@ _overrides: dict[str, object] = {}
 # Row quads (slk_spmm_quad) instead of slk_spmm where slk_quad_halves expects
 # them to be faster: layers of some 5% density and up at N of about 1000 and up,
 # all but the smallest where N is not a multiple of 4 (2304 x 768, N = 8192,
-# 20%: 219 -> 169 us; 3072 x 768, N = 1001, 10%: 82 -> 35; 4096^2 x 4096, 10%:
-# 540 -> 398). Below _QUAD_MIN_WORK live slots x N no shape gains (the smallest
+# 20%: 238 -> 190 us; 3072 x 768, N = 1001, 10%: 87 -> 37; 4096^2 x 4096, 10%:
+# 566 -> 462). Below _QUAD_MIN_WORK live slots x N no shape gains (the smallest
 # that does, 1152 x 384 at 10% and N = 1001, has 4.4e7), so the call is spared.
 _QUAD_MIN_WORK = 30_000_000
 
@@ -252,35 +255,66 @@ def _skew_slows_strips(W: PaddedCSR, N: int) -> bool:
     return (N % 4 == 0 or W.nnz * N < _SKEW_STRIP_MIN_WORK) and _skewed(W)
 
 
+# What quads and strips are taken for is kept with W's view, by N (dW: (N,)): it
+# depends on shape, capacity, live slots and the counts of heavy and dense rows,
+# which last as long as the view's row counts. Not while a kernel-choice knob is
+# forced, and not from a captured call, where the rows' skew may be unknown.
+_ROUTES = 64
+
+
+def _keep_route(routes: dict, key, choice):
+    if not _lib.FORCED_KNOBS and not torch.cuda.is_current_stream_capturing():
+        if len(routes) >= _ROUTES:
+            routes.clear()
+        routes[key] = choice
+    return choice
+
+
+def _quad_plan(W: PaddedCSR, K: int, N: int, mapped: bool = False):
+    """(halves, capturing, recorded) of the row quads to run W on a K x N X with;
+    None: slk_spmm. mapped: W is a cached transpose, run through its slot map."""
+    if _overrides:
+        halves = _overrides.get("quad")
+        if halves is not None:
+            capturing = torch.cuda.is_current_stream_capturing()
+            return (int(halves), capturing, not mapped) if halves else None
+        if "bin_shape" in _overrides or "spmm_phases" in _overrides:
+            return None
+    if W.nnz * N < _QUAD_MIN_WORK:
+        return None
+    view = W._view()
+    halves = view.routes.get(N)
+    if halves is None or _lib.FORCED_KNOBS:
+        halves = _lib.quad_halves(view, N)
+        if halves and _skew_slows_quads(W, N):
+            halves = 0
+        _keep_route(view.routes, N, halves)
+    if not halves:
+        return None
+    if not torch.cuda.is_current_stream_capturing():
+        return halves, False, False
+    if mapped or _spmm_scheduled(W, K, N):
+        return (halves, True, False) if W._has("_quads_kept", (halves, mapped)) else None
+    # (a graph cannot read the exact size of large quads, and would hold the bound)
+    if not _recording_pays(W, N) or _lib.quad_bytes(view, halves) > _lib.QUAD_READ_BYTES:
+        return None
+    return halves, True, True
+
+
 def _quad_halves(W: PaddedCSR, K: int, N: int, mapped: bool = False) -> int:
-    """64-column halves of the row quads (1 or 2) to run W on a K x N X with;
-    0: slk_spmm. mapped: W is a cached transpose, run through its slot map."""
-    forced = _overrides.get("quad")
-    if forced is not None:
-        return int(forced)
-    if W.nnz * N < _QUAD_MIN_WORK or "bin_shape" in _overrides or "spmm_phases" in _overrides:
-        return 0
-    halves = _lib.quad_halves(W._view(), N)
-    if not halves or _skew_slows_quads(W, N):
-        return 0
-    if torch.cuda.is_current_stream_capturing():
-        if mapped or _spmm_scheduled(W, K, N):
-            return halves if W._has("_quads_kept", (halves, mapped)) else 0
-        # (a graph cannot read the exact size of large quads, and would hold the bound)
-        if not _recording_pays(W, N) or _lib.quad_bytes(W._view(), halves) > _lib.QUAD_READ_BYTES:
-            return 0
-    return halves
+    """64-column halves (1 or 2) of _quad_plan's quads; 0: slk_spmm."""
+    plan = _quad_plan(W, K, N, mapped)
+    return plan[0] if plan else 0
 
 
-def _spmm_quads(W: PaddedCSR, values: torch.Tensor, X: torch.Tensor, Y: torch.Tensor,
-                halves: int, perm: torch.Tensor | None = None,
-                bias: torch.Tensor | None = None) -> bool:
+def _spmm_quads(W: PaddedCSR, values: torch.Tensor, X: torch.Tensor, Y: torch.Tensor, plan,
+                perm: torch.Tensor | None = None, bias: torch.Tensor | None = None) -> bool:
     """Y = W·X (+ bias) through W's row quads. False, with nothing launched and
     W's quads given up, where the memory for them is not to be had: slk_spmm needs
     none."""
-    recorded = perm is None and not _spmm_scheduled(W, *X.shape)
+    halves, capturing, recorded = plan
     try:
-        _lib.spmm_quad(W._view(), W._quads(halves, perm, recorded), values, X, Y, bias)
+        _lib.spmm_quad(W._view(), W._quads(halves, perm, capturing, recorded), values, X, Y, bias)
     except torch.OutOfMemoryError:
         W._quads_kept = (-1, {})
         return False
@@ -315,14 +349,12 @@ def _spmm_view(W: PaddedCSR, X: torch.Tensor):
 
 
 def _launch_spmm(W: PaddedCSR, X: torch.Tensor, bias: torch.Tensor | None = None,
-                 halves: int | None = None) -> torch.Tensor:
-    """W·X (+ bias per row); halves: what _quad_halves said, if it was asked."""
+                 quads: bool = True) -> torch.Tensor:
+    """W·X (+ bias per row); quads: not known to be out of the question."""
     Y = torch.empty((W.nrows, X.shape[1]), dtype=torch.float32, device=X.device)
-    if halves is None:
-        halves = _quad_halves(W, *X.shape)
-    if halves and _spmm_quads(W, W.values, X, Y, halves, bias=bias):
-        return Y
-    _lib.spmm(_spmm_view(W, X), X, Y, bias)
+    plan = _quad_plan(W, *X.shape) if quads else None
+    if plan is None or not _spmm_quads(W, W.values, X, Y, plan, bias=bias):
+        _lib.spmm(_spmm_view(W, X), X, Y, bias)
     return Y
 
 
@@ -383,44 +415,61 @@ def _sddmm_scheduled(W: PaddedCSR, N: int) -> bool:
 
 # Strips (slk_sddmm_strips) instead of slk_sddmm where slk_strip_choose expects
 # them to be faster: N not a multiple of 4 (1537 x 1000 at 20%, N = 1777: 194 ->
-# 56 us), N below 1024 or too few slots for the segment list (512 x 784 at 20%, N
-# = 8192: 159 -> 108), and layers around 3-5% and 20-40% (4096^2 x 4096 at 5%: 585
-# -> 380; 2304 x 768 at 30%, N = 8192: 373 -> 280). Below _STRIP_MIN_WORK live
+# 52 us), N below 1024 or too few slots for the segment list (512 x 784 at 20%, N
+# = 8192: 159 -> 108), and layers around 3-5% and 20-40% (4096^2 x 4096 at 5%: 579
+# -> 405; 2304 x 768 at 30%, N = 8192: 365 -> 283). Below _STRIP_MIN_WORK live
 # slots x N no shape gains.
 _STRIP_MIN_WORK = 30_000_000
 
 
-def _strip_sizes(W: PaddedCSR, N: int):
-    """(block, slots, per_wave, parts) of the strips to run W's dW with at N
-    columns; None: slk_sddmm."""
-    if "strips" in _overrides:
-        return _overrides["strips"]
-    if W.nnz * N < _STRIP_MIN_WORK or "seg" in _overrides or "dense_dw" in _overrides or \
+def _strip_plan(W: PaddedCSR, N: int):
+    """((block, slots, per_wave, parts), capturing, recorded) of the strips to run
+    W's dW with at N columns; None: slk_sddmm."""
+    if _overrides:
+        if "strips" in _overrides:
+            sizes = _overrides["strips"]
+            return (sizes, torch.cuda.is_current_stream_capturing(), True) if sizes else None
+        if "seg" in _overrides or "dense_dw" in _overrides:
+            return None
+    if W.nnz * N < _STRIP_MIN_WORK or \
             not _lib.FORCED_KNOBS.isdisjoint(("sddmm_g", "seg_lean", "seg_group")):
         return None
-    sizes = W._strip_choice(N)
-    if not sizes or _skew_slows_strips(W, N):
+    view = W._view()
+    sizes = view.routes.get((N,))
+    if sizes is None:
+        sizes = _lib.strip_choose(view, N)[0] or ()
+        if sizes and _skew_slows_strips(W, N):
+            sizes = ()
+        _keep_route(view.routes, (N,), sizes)
+    if not sizes:
         return None
-    if torch.cuda.is_current_stream_capturing():
-        if not (W._has("_strips_kept", sizes) if _sddmm_scheduled(W, N) else _recording_pays(W, N)):
-            return None
-    return sizes
+    if not torch.cuda.is_current_stream_capturing():
+        return sizes, False, False
+    if _sddmm_scheduled(W, N):
+        return (sizes, True, False) if W._has("_strips_kept", sizes) else None
+    return (sizes, True, True) if _recording_pays(W, N) else None
+
+
+def _strip_sizes(W: PaddedCSR, N: int):
+    """_strip_plan's (block, slots, per_wave, parts); None: slk_sddmm."""
+    plan = _strip_plan(W, N)
+    return plan[0] if plan else None
 
 
 def _launch_sddmm(W: PaddedCSR, dY: torch.Tensor, X: torch.Tensor, kernel: str,
                   dbias: torch.Tensor | None = None) -> torch.Tensor:
     dW = torch.empty(W.total_capacity, dtype=torch.float32, device=X.device)
-    order = _lib.SLK_DW_SCALAR if kernel == "scalar" else _lib.SLK_DW_SIMD
-    sizes = _strip_sizes(W, X.shape[1]) if order == _lib.SLK_DW_SIMD else None
-    if sizes:
+    if kernel == "scalar":
+        _lib.sddmm(W._view(), dY, X, dW, _lib.SLK_DW_SCALAR, dbias)
+        return dW
+    plan = _strip_plan(W, X.shape[1])
+    if plan is not None:
         try:
-            strips = W._strips(sizes, not _sddmm_scheduled(W, X.shape[1]))
-            _lib.sddmm_strips(W._view(), strips, dY, X, dW, dbias)
+            _lib.sddmm_strips(W._view(), W._strips(*plan), dY, X, dW, dbias)
             return dW
         except torch.OutOfMemoryError:  # for the strips or their copy of X
             W._strips_kept = (-1, {})
-    view = _sddmm_view(W, X) if order == _lib.SLK_DW_SIMD else W._view()
-    _lib.sddmm(view, dY, X, dW, order, dbias)
+    _lib.sddmm(_sddmm_view(W, X), dY, X, dW, _lib.SLK_DW_SIMD, dbias)
     return dW
 
 
@@ -503,14 +552,15 @@ def _spmm_backward(W: PaddedCSR, X: torch.Tensor, dY_f32: torch.Tensor, kernel: 
         dW_values = _launch_sddmm(W, dY_f32, _device_f32(X), kernel, dbias)
     if need_dx:
         WT, perm, fresh = _transpose_entry(W)
-        halves = _quad_halves(WT, *dY_f32.shape, mapped=True)
-        if halves:  # through W's values: no refresh of WT's
+        plan = _quad_plan(WT, *dY_f32.shape, mapped=True)
+        if plan is not None:  # through W's values: no refresh of WT's
             dX = torch.empty((W.ncols, dY_f32.shape[1]), dtype=torch.float32, device=W.device)
-        if not halves or not _spmm_quads(WT, W.values, dY_f32, dX, halves, perm):
-            dX = None
+            if not _spmm_quads(WT, W.values, dY_f32, dX, plan, perm):
+                dX = None
+        if dX is None:
             if not fresh:
                 _lib.transpose_refresh(W.values, perm, WT.values)
-            dX = _launch_spmm(WT, dY_f32, halves=0)
+            dX = _launch_spmm(WT, dY_f32, quads=False)
     return dW_values, dX
 
 

@@ -51,7 +51,7 @@ def test_forward_dw_and_dx_run_without_schedules(calls, monkeypatch):
 
 def test_a_refused_value_buffer_gives_the_kept_quads_up(calls, monkeypatch):
     W = from_oracle(oracle.uniform_rows(40, 30, 9, seed=1))
-    monkeypatch.setattr(layout.PaddedCSR, "_quads", lambda *a: "quads")
+    monkeypatch.setattr(layout.PaddedCSR, "_quads", lambda *a: object())
     monkeypatch.setattr(_lib, "spmm_quad", _lib.quad_build)
     W._quads_kept = (W.topology_version, {(1, False): "kept"})
     ops._launch_spmm(W, torch.zeros(30, 8))
@@ -68,5 +68,6 @@ def test_large_quads_are_not_recorded_in_graphs(monkeypatch):
     monkeypatch.setattr(layout.PaddedCSR, "nnz", property(lambda W: 1 << 24))
     monkeypatch.setattr(layout.PaddedCSR, "_skewed", lambda W: False)
     for view, takes in ((v, 0), (small, 2)):
+        view.routes = {}
         monkeypatch.setattr(layout.PaddedCSR, "_view", lambda W: view)
         assert ops._quad_halves(W, view.ncols, 8192) == takes

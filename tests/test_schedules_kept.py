@@ -53,21 +53,23 @@ def W():
     return layout.from_dense(torch.eye(4))
 
 
-def _build(made):
-    def build():
+def _get(W, gpu, made, name, key, recorded=False):
+    """What the schedules of layout.PaddedCSR do: find, else build and keep."""
+    a = W._find(name, key, gpu.capturing, recorded)
+    if a is None:
         a = _Array()
         made.append(a)
-        return a, (a,)
-    return build
+        W._keep(name, key, a, (a,), gpu.capturing)
+    return a
 
 
 def test_another_stream_waits_for_the_build_and_is_a_user_of_its_arrays(W, gpu):
     made = []
-    first = W._kept("_quads_kept", 1, _build(made))
-    assert W._kept("_quads_kept", 1, _build(made)) is first and gpu.log == []
+    first = _get(W, gpu, made, "_quads_kept", 1)
+    assert _get(W, gpu, made, "_quads_kept", 1) is first and gpu.log == []
     for stream in (2, 3, 2, 1):
         gpu.stream = stream
-        assert W._kept("_quads_kept", 1, _build(made)) is first and len(made) == 1
+        assert _get(W, gpu, made, "_quads_kept", 1) is first and len(made) == 1
     assert gpu.log == [("record", 1), ("wait", 2, "event of 1"),
                        ("record", 1), ("wait", 3, "event of 1")]
     assert first.users == [2, 3]
@@ -77,39 +79,39 @@ def test_every_key_of_a_topology_is_kept(W, gpu):
     """Nothing built for this topology is dropped while it lasts: a captured
     call may hold its address."""
     made = []
-    got = [W._kept("_strips_kept", n, _build(made)) for n in range(8)]
-    assert [W._kept("_strips_kept", n, _build(made)) for n in range(8)] == got and len(made) == 8
+    got = [_get(W, gpu, made, "_strips_kept", n) for n in range(8)]
+    assert [_get(W, gpu, made, "_strips_kept", n) for n in range(8)] == got and len(made) == 8
     W.rewrite_row(0, [1], [1.0])
-    assert W._kept("_strips_kept", 0, _build(made)) is not got[0]
+    assert _get(W, gpu, made, "_strips_kept", 0) is not got[0]
 
 
 def test_a_capture_pins_what_it_reads_until_one_under_a_newer_topology(W, gpu):
     made = []
-    old = W._kept("_segs_kept", 1, _build(made))
+    old = _get(W, gpu, made, "_segs_kept", 1)
     gpu.capturing, gpu.stream = True, 2
-    assert W._kept("_segs_kept", 1, _build(made)) is old
-    assert W._kept("_segs_kept", 1, _build(made)) is old
+    assert _get(W, gpu, made, "_segs_kept", 1) is old
+    assert _get(W, gpu, made, "_segs_kept", 1) is old
     assert gpu.log == [], "no wait for an event of before the capture"
     assert [b.value for b in W._pinned[1]] == [old]
     gpu.capturing, gpu.stream = False, 1
     W.rewrite_row(0, [1], [1.0])
-    new = W._kept("_segs_kept", 1, _build(made))
+    new = _get(W, gpu, made, "_segs_kept", 1)
     assert new is not old and [b.value for b in W._pinned[1]] == [old]
     gpu.capturing = True
-    W._kept("_segs_kept", 1, _build(made))
+    _get(W, gpu, made, "_segs_kept", 1)
     assert [b.value for b in W._pinned[1]] == [new]
 
 
 def test_what_a_capture_builds_is_the_graphs_alone(W, gpu):
     made = []
     gpu.capturing = True
-    W._kept("_phases_kept", 1, _build(made))
+    _get(W, gpu, made, "_phases_kept", 1)
     gpu.capturing = False
-    W._kept("_phases_kept", 1, _build(made))
+    _get(W, gpu, made, "_phases_kept", 1)
     assert len(made) == 2
     # recorded: anew under capture though a kept one is there, which stays
-    kept = W._kept("_quads_kept", 1, _build(made), recorded=True)
+    kept = _get(W, gpu, made, "_quads_kept", 1, recorded=True)
     gpu.capturing = True
-    assert W._kept("_quads_kept", 1, _build(made), recorded=True) is not kept
+    assert _get(W, gpu, made, "_quads_kept", 1, recorded=True) is not kept
     gpu.capturing = False
-    assert W._kept("_quads_kept", 1, _build(made), recorded=True) is kept and len(made) == 4
+    assert _get(W, gpu, made, "_quads_kept", 1, recorded=True) is kept and len(made) == 4
